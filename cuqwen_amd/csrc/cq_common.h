@@ -173,6 +173,7 @@ constexpr double kWeightSigma = 0.02;
 // ------------------------------------------------------------ quantization
 constexpr int kGroup = 128;
 constexpr int kMaxHeadDim = 128;
+constexpr int kNumCUs = 256;   // MI355X
 
 // ----------------------------------------------------------- KV cache tiles
 // Per (layer, kv head) the cache holds max_seq_len slots.  K is stored in

@@ -1029,6 +1029,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       at.max_seq = c.max_seq_len;
       at.kcache8 = kc8; at.vcache8 = vc8; at.kscale = ksc; at.vscale = vsc; at.kv_fmt = s->kv_dtype;
       at.int4_layout = c.quant_type == CQ_QUANT_INT4;
+      at.part = s->pf_part; at.part_bytes = kPrefillPartBytes;
       CQ_TRY(launch_pf_attention(at, st));
       if (l == c.n_layers - 1) {   // only the last token's row goes on
         if (c0 + M == n) CQ_TRY(prefill_tail(s, M));

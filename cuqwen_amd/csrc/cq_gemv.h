@@ -124,7 +124,6 @@ template <int Q> __device__ __forceinline__ float plane_order_packed(const u4_t&
 // Building blocks of the GEMV kernels: input staging, weight steps, row
 // mapping and epilogues.
 
-constexpr int kNumCUs = 256;   // MI355X
 
 template <int Q> __device__ __forceinline__ constexpr bool quantized() { return Q != CQ_QUANT_FP16; }
 

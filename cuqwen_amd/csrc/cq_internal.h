@@ -177,6 +177,10 @@ struct PfAttnArgs {
   const float* vscale = nullptr;
   int kv_fmt = CQ_KV_INT8;
   bool int4_layout = false;   // out in the int4 GEMM input layout (else natural order)
+  // fp32 workspace for the partials of a key range split over blocks (nullptr: no split)
+  float* part = nullptr;
+  size_t part_bytes = 0;
+  int n_rb = 0, splits = 1;   // set by the launcher: row blocks per kv head, key ranges
 };
 int launch_pf_norm(const __half* x, const __half* w, float eps, int M, int dim, __half* A, float* inv, int quant,
                    hipStream_t stream);

@@ -26,6 +26,7 @@
 // int8 / fp16: natural), so neither operand needs a shuffle in the main loop.
 #include "cq_attention.h"
 #include "cq_gemv.h"
+#include "cq_prefill.h"
 
 #include <algorithm>
 #include <type_traits>
@@ -36,23 +37,6 @@ constexpr int kPfWaves = 8;
 constexpr int kPfThreads = kPfWaves * 64;
 constexpr int kPfK = 128;         // K per main-loop step (one quantization group)
 constexpr int kPfMaxSplit = 8;
-
-// Activation layout of the GEMM inputs, chosen by the weights' format so the
-// A operand needs no shuffle: int4 stores each 8-group in the order
-// [0,4,1,5,2,6,3,7] with the odd elements divided by 16 (the unpack yields the
-// odd nibbles as 16 n without a shift); int8 and fp16 keep natural order.
-__device__ __forceinline__ int pf_pos(int k, bool int4) {
-  if (!int4) return k;
-  const int e = k & 7;
-  return (k & ~7) | (e < 4 ? 2 * e : 2 * e - 7);
-}
-// value stored for element k.  The /16 is a power-of-two scale, exact for
-// |v| >= 2^-10; below that v/16 falls in fp16's subnormal range and keeps
-// fewer bits (at most 2^-21 absolute error on the element: half the 2^-24
-// subnormal spacing, times 16).
-__device__ __forceinline__ _Float16 pf_val(float v, int k, bool int4) {
-  return (_Float16)((int4 && (k & 1)) ? v * 0.0625f : v);
-}
 
 // ------------------------------------------------------------- row norm
 // RMSNorm of one token row by one block (dim a multiple of 8): A row =
@@ -744,301 +728,6 @@ __global__ __launch_bounds__(kPfQkvThreads) void pf_split_qkv(const PfGemmArgs a
   }
 }
 
-// ------------------------------------------------------ causal attention
-// Block = (16 consecutive tokens, one query head): the 16 tokens are the
-// columns of S^T = K Q^T; 8 waves take every 8th 32-key tile up to the last
-// token's position (double-buffered like the decode kernel), keys past a
-// token's own position are masked per column, and the waves merge in LDS.
-// Output rows are written in the GEMM activation layout.
-template <int HD>
-__device__ __forceinline__ void pf_attend_tile(KVTile<HD>& t, const h8_t* qb, int ti, int t_lane, int t_max,
-                                               float scale, int j, float& m, float& l, f4_t* o) {
-  constexpr int KK = HD / 32, DT = HD / 16;
-  f4_t s[2];
-#pragma unroll
-  for (int st = 0; st < 2; ++st) {
-    s[st] = f4_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int kk = 0; kk < KK; ++kk) s[st] = __builtin_amdgcn_mfma_f32_16x16x32_f16(t.ka[st][kk], qb[kk], s[st], 0, 0, 0);
-  }
-  const int key0 = ti * kTileKeys + 4 * j;
-  float sv[8];
-  float mt = -INFINITY;
-#pragma unroll
-  for (int st = 0; st < 2; ++st)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      float v = (float)(_Float16)(s[st][i] * scale);   // kernels.cu:171
-      if (key0 + st * 16 + i >= t_lane) v = -INFINITY;
-      sv[st * 4 + i] = v;
-      mt = fmaxf(mt, v);
-    }
-  mt = fmaxf(mt, __shfl_xor(mt, 16, kWave));
-  mt = fmaxf(mt, __shfl_xor(mt, 32, kWave));
-  const float mn = fmaxf(m, mt);
-  // a column can have no valid key yet (its token precedes this tile)
-  const float alpha = m == -INFINITY ? 0.f : __expf(m - mn);
-  m = mn;
-  l *= alpha;
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] *= alpha;
-  h8_t pb;
-#pragma unroll
-  for (int e = 0; e < 8; ++e) {
-    const float p = sv[e] == -INFINITY ? 0.f : __expf(sv[e] - mn);
-    l += p;
-    pb[e] = (_Float16)p;
-  }
-  if ((ti + 1) * kTileKeys > t_max) {
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const int key = ti * kTileKeys + (e < 4 ? 4 * j + e : 16 + 4 * j + e - 4);
-        if (key >= t_max) t.va[dt][e] = (_Float16)0.f;
-      }
-  }
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(t.va[dt], pb, o[dt], 0, 0, 0);
-}
-
-template <int HD, int KV8>   // KV8: 0 fp16 cache, else the code format of the quantized cache
-__global__ __launch_bounds__(kAttnThreads) void pf_attention_kernel(const PfAttnArgs a) {
-  constexpr int KK = HD / 32, DT = HD / 16;
-  const int t0 = blockIdx.x * 16, hq = blockIdx.y;
-  const int g = a.n_heads / a.n_kv, kvh = hq / g;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int h = lane & 15, j = lane >> 4;   // h: token column
-  const int tcol = min(t0 + h, a.M - 1);
-  const int t_lane = a.pos0 + tcol + 1;                       // keys visible to this column
-  const int t_max = a.pos0 + min(t0 + 16, a.M);               // keys visible to the block
-  const int n_tiles = (t_max + kTileKeys - 1) / kTileKeys;
-  const float scale = 1.0f / sqrtf((float)HD);
-  const _Float16* kbase = a.kcache + (int64_t)kvh * a.max_seq * HD;
-  const _Float16* vbase = a.vcache + (int64_t)kvh * a.max_seq * HD;
-  h8_t qb[KK];
-  const _Float16* q = a.q + (int64_t)tcol * a.n_heads * HD + hq * HD;
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) qb[kk] = __builtin_bit_cast(h8_t, load_u4(q + kk * 32 + j * 8));
-  float m = -INFINITY, l = 0.f;
-  f4_t o[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = f4_t{0.f, 0.f, 0.f, 0.f};
-  int ti = wave;
-  if constexpr (KV8) {
-    const int8_t* kb8 = a.kcache8 + (int64_t)kvh * a.max_seq * HD;
-    const int8_t* vb8 = a.vcache8 + (int64_t)kvh * a.max_seq * HD;
-    const float* ksc = a.kscale + (int64_t)kvh * a.max_seq;
-    const float* vsc = a.vscale + (int64_t)kvh * a.max_seq;
-    const uint32_t magic = vgpr_const(0x64646464u);
-    KVTile8<HD> A, B;
-    if (ti < n_tiles) load_tile8<HD>(A, kb8, vb8, ksc, vsc, ti, lane);
-    for (; ti < n_tiles; ti += 2 * kAttnWaves) {
-      const int t1 = ti + kAttnWaves;
-      if (t1 < n_tiles) load_tile8<HD>(B, kb8, vb8, ksc, vsc, t1, lane);
-      attend_tile8<HD, KV8>(A, qb, ti, t_lane, scale, j, m, l, o, magic);
-      if (t1 >= n_tiles) break;
-      if (t1 + kAttnWaves < n_tiles) load_tile8<HD>(A, kb8, vb8, ksc, vsc, t1 + kAttnWaves, lane);
-      attend_tile8<HD, KV8>(B, qb, t1, t_lane, scale, j, m, l, o, magic);
-    }
-  } else {
-    KVTile<HD> A, B;
-    if (ti < n_tiles) load_tile<HD>(A, kbase, vbase, ti, lane);
-    for (; ti < n_tiles; ti += 2 * kAttnWaves) {
-      const int t1 = ti + kAttnWaves;
-      if (t1 < n_tiles) load_tile<HD>(B, kbase, vbase, t1, lane);
-      pf_attend_tile<HD>(A, qb, ti, t_lane, t_max, scale, j, m, l, o);
-      if (t1 >= n_tiles) break;
-      if (t1 + kAttnWaves < n_tiles) load_tile<HD>(A, kbase, vbase, t1 + kAttnWaves, lane);
-      pf_attend_tile<HD>(B, qb, t1, t_lane, t_max, scale, j, m, l, o);
-    }
-  }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-
-  __shared__ float wm[kAttnWaves][16], wl[kAttnWaves][16];
-  __shared__ float wo[kAttnWaves][16][HD + 1];
-  if (j == 0) { wm[wave][h] = m; wl[wave][h] = l; }
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) wo[wave][h][dt * 16 + 4 * j + i] = o[dt][i];
-  __syncthreads();
-  const int qd = a.n_heads * HD;
-  for (int idx = threadIdx.x; idx < 16 * HD; idx += kAttnThreads) {
-    const int c = idx / HD, d = idx % HD;
-    if (t0 + c >= a.M) continue;
-    float M = -INFINITY;
-#pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) M = fmaxf(M, wm[w][c]);
-    float L = 0.f, O = 0.f;
-#pragma unroll
-    for (int w = 0; w < kAttnWaves; ++w) {
-      const float f = wm[w][c] == -INFINITY ? 0.f : __expf(wm[w][c] - M);
-      L += wl[w][c] * f;
-      O += wo[w][c][d] * f;
-    }
-    const int k = hq * HD + d;
-    a.out[(int64_t)(t0 + c) * qd + pf_pos(k, a.int4_layout)] =
-        pf_val((float)(_Float16)(O * (1.0f / (L + 1e-9f))), k, a.int4_layout);
-  }
-}
-
-// Causal attention with the K / V tiles shared by the query heads of a GQA
-// group (fp16 cache): block = (16 consecutive tokens, one kv head), 16 waves:
-// wave w owns query head kvh * g + (w % 8) and, with its partner w ^ 8, runs
-// the online softmax over every key tile up to the block's last token (even
-// tiles in waves 0-7, odd tiles in waves 8-15); the two halves merge in LDS
-// at the end.  The tiles stream global -> registers -> LDS (a tile's K and V
-// are each one contiguous 32-key block of the tiled cache), a pair of tiles
-// per stage, two stages, and every head of the group reads them from LDS:
-// the cache is read once per kv head instead of once per query head.
-constexpr int kPfGqaWaves = 16;
-template <int HD>
-__global__ __launch_bounds__(kPfGqaWaves * kWave) void pf_attention_gqa_kernel(const PfAttnArgs a) {
-  constexpr int KK = HD / 32, DT = HD / 16;
-  constexpr int TILE = kTileKeys * HD;               // halves of K (or V) per tile
-  constexpr int STAGE = 4 * TILE;                    // two tiles, K and V
-  constexpr int CHUNKS = STAGE * 2 / 1024;           // 1 KB pieces per stage
-  constexpr int PER_WAVE = (CHUNKS + kPfGqaWaves - 1) / kPfGqaWaves;
-  constexpr int MERGE = 8 * kWave * (2 + 4 * DT);    // floats of one half's softmax state
-  constexpr int SM = 2 * STAGE > 2 * MERGE ? 2 * STAGE : 2 * MERGE;
-  __shared__ __align__(16) _Float16 st[SM];
-  const int t0 = blockIdx.x * 16, kvh = blockIdx.y;
-  const int g = a.n_heads / a.n_kv;
-  const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
-  const int head = wave & 7, half = wave >> 3;
-  const int h = lane & 15, j = lane >> 4;   // h: token column
-  const int t_max = a.pos0 + min(t0 + 16, a.M);   // keys visible to the block
-  const int n_tiles = (t_max + kTileKeys - 1) / kTileKeys;
-  const int n_steps = (n_tiles + 1) / 2;
-  const _Float16* kbase = a.kcache + (int64_t)kvh * a.max_seq * HD;
-  const _Float16* vbase = a.vcache + (int64_t)kvh * a.max_seq * HD;
-  // A step's tile pair goes global -> registers one step ahead, then into
-  // one of two LDS stages at the start of the step that reads it.  Stage
-  // layout: [tile 0: K, V][tile 1: K, V]; piece c of a stage is 1 KB (the
-  // pair's second tile may be past the end).
-  u4_t kv[PER_WAVE];
-  auto piece = [&](int i, int step, int* tt, bool* isv, int* cc) {
-    const int c = i * kPfGqaWaves + wave;
-    *tt = c / (CHUNKS / 2);
-    const int r = c % (CHUNKS / 2);
-    *isv = r >= CHUNKS / 4;
-    *cc = *isv ? r - CHUNKS / 4 : r;
-    return c < CHUNKS && 2 * step + *tt < n_tiles;
-  };
-  auto load = [&](int step) {
-#pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i) {
-      int tt, cc;
-      bool isv;
-      if (piece(i, step, &tt, &isv, &cc))
-        kv[i] = load_u4((isv ? vbase : kbase) + (int64_t)(2 * step + tt) * TILE + cc * 512 + lane * 8);
-    }
-  };
-  auto store = [&](int step) {
-    _Float16* dst = st + (step & 1) * STAGE;
-#pragma unroll
-    for (int i = 0; i < PER_WAVE; ++i) {
-      int tt, cc;
-      bool isv;
-      if (piece(i, step, &tt, &isv, &cc))
-        *reinterpret_cast<u4_t*>(dst + tt * 2 * TILE + (isv ? TILE : 0) + cc * 512 + lane * 8) = kv[i];
-    }
-  };
-  const bool active = head < g;
-  const int hq = kvh * g + min(head, g - 1);
-  const int tcol = min(t0 + h, a.M - 1);
-  const int t_lane = a.pos0 + tcol + 1;                // keys visible to this column
-  h8_t qb[KK];
-  const _Float16* q = a.q + (int64_t)tcol * a.n_heads * HD + hq * HD;
-#pragma unroll
-  for (int kk = 0; kk < KK; ++kk) qb[kk] = __builtin_bit_cast(h8_t, load_u4(q + kk * 32 + j * 8));
-  load(0);
-  const float scale = 1.0f / sqrtf((float)HD);
-  float m = -INFINITY, l = 0.f;
-  f4_t o[DT];
-#pragma unroll
-  for (int dt = 0; dt < DT; ++dt) o[dt] = f4_t{0.f, 0.f, 0.f, 0.f};
-  for (int sp = 0; sp < n_steps; ++sp) {
-    // this step's pieces (loaded during the previous step) into LDS stage
-    // sp % 2, last read at step sp - 2, which every wave finished before the
-    // previous barrier; then visible to all waves
-    __builtin_amdgcn_s_waitcnt(0x0F70);
-    store(sp);
-    __builtin_amdgcn_s_waitcnt(0xC07F);
-    lds_barrier();
-    if (sp + 1 < n_steps) load(sp + 1);
-    const int ti = 2 * sp + half;
-    if (active && ti < n_tiles) {
-      const _Float16* kt = st + (sp & 1) * STAGE + half * 2 * TILE;
-      const _Float16* vt = kt + TILE;
-      KVTile<HD> A;
-#pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-#pragma unroll
-        for (int kk = 0; kk < KK; ++kk)
-          A.ka[s2][kk] = *reinterpret_cast<const h8_t*>(kt + s2 * 16 * HD + (kk * 64 + lane) * 8);
-#pragma unroll
-      for (int dt = 0; dt < DT; ++dt) A.va[dt] = *reinterpret_cast<const h8_t*>(vt + (dt * 64 + lane) * 8);
-      pf_attend_tile<HD>(A, qb, ti, t_lane, t_max, scale, j, m, l, o);
-    }
-  }
-  l += __shfl_xor(l, 16, kWave);
-  l += __shfl_xor(l, 32, kWave);
-  // merge the odd-tile half into the even one (over the stage buffers)
-  __syncthreads();
-  float* mg = reinterpret_cast<float*>(st) + head * kWave * (2 + 4 * DT);
-  if (half == 1 && active) {
-    mg[lane] = m;
-    mg[kWave + lane] = l;
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) mg[(2 + 4 * dt + i) * kWave + lane] = o[dt][i];
-  }
-  __syncthreads();
-  // the merged rows go through LDS (over the merge area, once every wave
-  // has read it) so each token's g heads are written as one contiguous run
-  // of 16-byte pieces
-  const bool writer = half == 0 && active;
-  float ov[DT][4];
-  if (writer) {
-    const float m1 = mg[lane], l1 = mg[kWave + lane];
-    const float M = fmaxf(m, m1);
-    const float f0 = m == -INFINITY ? 0.f : __expf(m - M), f1 = m1 == -INFINITY ? 0.f : __expf(m1 - M);
-    const float inv = 1.0f / (l * f0 + l1 * f1 + 1e-9f);
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) ov[dt][i] = (o[dt][i] * f0 + mg[(2 + 4 * dt + i) * kWave + lane] * f1) * inv;
-  }
-  __syncthreads();
-  const int GW = g * HD;   // output halves per token of this kv head
-  // [16 tokens][GW + 8]: the 16-byte pad moves consecutive token rows to
-  // different bank groups (unpadded, the row stride is a multiple of the
-  // 256-byte bank row and the 16 token columns' 2-byte stores collide)
-  const int OS = GW + 8;
-  _Float16* ot = st;
-  if (writer) {
-#pragma unroll
-    for (int dt = 0; dt < DT; ++dt)
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int k = head * HD + dt * 16 + 4 * j + i;   // head * HD is a multiple of 8: the layout stays in the tile
-        ot[h * OS + pf_pos(k, a.int4_layout)] = pf_val((float)(_Float16)ov[dt][i], k, a.int4_layout);
-      }
-  }
-  __syncthreads();
-  const int qd = a.n_heads * HD;
-  for (int idx = threadIdx.x; idx < 16 * (GW / 8); idx += kPfGqaWaves * kWave) {
-    const int c = idx / (GW / 8), p8 = idx % (GW / 8);
-    if (t0 + c < a.M)
-      *reinterpret_cast<u4_t*>(a.out + (int64_t)(t0 + c) * qd + kvh * GW + 8 * p8) =
-          *reinterpret_cast<const u4_t*>(ot + c * OS + 8 * p8);
-  }
-}
-
 // One row of a GEMM input back to natural order (the int4 layout stores each
 // 8-group as [0,4,1,5,2,6,3,7] with the odd elements / 16; the scale is a
 // power of two, so the round trip is exact for odd elements of magnitude at
@@ -1156,31 +845,6 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream) {
     case CQ_QUANT_INT8: return launch_pf_gemm_q<CQ_QUANT_INT8>(a, stream);
     default: return launch_pf_gemm_q<CQ_QUANT_INT4>(a, stream);
   }
-}
-
-int launch_pf_attention(const PfAttnArgs& a, hipStream_t stream) {
-  if (a.head_dim != 64 && a.head_dim != 128) return fail(CQ_EINVAL, "prefill attention: head_dim must be 64 or 128");
-  if (a.M <= 0 || a.pos0 < 0 || a.pos0 + a.M > a.max_seq) return fail(CQ_ERANGE, "prefill attention: positions");
-  const dim3 grid((a.M + 15) / 16, a.n_heads);
-  if (a.kcache8) {
-    if (!a.vcache8 || !a.kscale || !a.vscale) return fail(CQ_EINVAL, "prefill attention: quantized cache pointers");
-    if (a.kv_fmt == CQ_KV_FP8) {
-      if (a.head_dim == 128) hipLaunchKernelGGL((pf_attention_kernel<128, CQ_KV_FP8>), grid, dim3(kAttnThreads), 0, stream, a);
-      else hipLaunchKernelGGL((pf_attention_kernel<64, CQ_KV_FP8>), grid, dim3(kAttnThreads), 0, stream, a);
-    } else {
-      if (a.head_dim == 128) hipLaunchKernelGGL((pf_attention_kernel<128, CQ_KV_INT8>), grid, dim3(kAttnThreads), 0, stream, a);
-      else hipLaunchKernelGGL((pf_attention_kernel<64, CQ_KV_INT8>), grid, dim3(kAttnThreads), 0, stream, a);
-    }
-  } else if (a.n_heads / a.n_kv <= 8) {
-    const dim3 g2((a.M + 15) / 16, a.n_kv);
-    if (a.head_dim == 128) hipLaunchKernelGGL((pf_attention_gqa_kernel<128>), g2, dim3(kPfGqaWaves * kWave), 0, stream, a);
-    else hipLaunchKernelGGL((pf_attention_gqa_kernel<64>), g2, dim3(kPfGqaWaves * kWave), 0, stream, a);
-  } else {
-    if (a.head_dim == 128) hipLaunchKernelGGL((pf_attention_kernel<128, 0>), grid, dim3(kAttnThreads), 0, stream, a);
-    else hipLaunchKernelGGL((pf_attention_kernel<64, 0>), grid, dim3(kAttnThreads), 0, stream, a);
-  }
-  CQ_HIP(hipGetLastError());
-  return CQ_OK;
 }
 
 }  // namespace cq

@@ -153,6 +153,63 @@ def test_prefill_matches_decode_real_shapes(model, quant, layers, n, n_ctx):
     w.free()
 
 
+# query rows (n * group) around the 32-row waves and the 64 / 128 / 256-row
+# blocks, contexts around the 32-key tiles and long enough for split key
+# ranges (2 tokens at 3001: more ranges than a block has waves), every cache
+# format, both head sizes, groups that do not divide a wave
+@pytest.mark.parametrize("heads,kv_heads,hd,n,pos0", [
+    (14, 2, 64, 9, 0), (14, 2, 64, 37, 31), (14, 2, 64, 5, 1000), (16, 16, 64, 33, 0), (28, 4, 128, 2, 3001),
+    (28, 4, 128, 10, 0), (28, 4, 128, 37, 95), (12, 1, 128, 11, 700), (16, 1, 128, 17, 33), (5, 5, 128, 64, 32)])
+@pytest.mark.parametrize("kv", [cq.KV_FP16, cq.KV_INT8, cq.KV_FP8])
+def test_prefill_attention_edges_match_decode(heads, kv_heads, hd, n, pos0, kv):
+    cfg = tiny_config(2, n_heads=heads, n_kv_heads=kv_heads, head_dim=hd, dim=512, max_seq_len=4096)
+    w = cq.synth_weights(cfg, 11)
+    prompt = _prompt(cfg, n, 3)
+    st, ref = cq.State(cfg, w, kv_dtype=kv), cq.State(cfg, w, kv_dtype=kv)
+    if pos0:
+        st.fill_kv(pos0, 5)
+        ref.fill_kv(pos0, 5)
+    st.prefill(prompt, pos0)
+    for i, t in enumerate(prompt):
+        ref.forward(t, pos0 + i, [])
+    assert _rel(st.logits(), ref.logits()) <= TOL
+    # layer 1's rows come from layer 0's attention of every token; a quantized
+    # row may differ by a code (int8: 1/127 of its maximum, E4M3: 0.08)
+    tol = {cq.KV_FP16: TOL, cq.KV_INT8: 2e-2, cq.KV_FP8: 0.08}[kv]
+    for h in range(kv_heads):
+        for kind in (0, 1):
+            a, b = (x.kv_read(1, h, kind, pos0 + n)[pos0:] for x in (st, ref))
+            assert _rel(a, b) <= tol, (h, kind)
+    st.free()
+    ref.free()
+    w.free()
+
+
+@pytest.mark.parametrize("hd,n,pos0", [(64, 40, 0), (128, 3, 600), (128, 33, 5)])
+def test_prefill_ignores_stale_cache(hd, n, pos0):
+    """Whatever the cache holds past the context (NaN here) stays out of the
+    result, bit for bit."""
+    cfg = tiny_config(0, n_heads=4, n_kv_heads=2, head_dim=hd, max_seq_len=1024)
+    w = cq.synth_weights(cfg, 12)
+    prompt = _prompt(cfg, n, 4)
+    out = []
+    for stale in (False, True):
+        st = cq.State(cfg, w)
+        if stale:
+            bad = np.full((1024, hd), np.nan, dtype=np.float16)
+            for layer in range(cfg.n_layers):
+                for h in range(2):
+                    for kind in (0, 1):
+                        st.kv_write(layer, h, kind, bad)
+        if pos0:
+            st.fill_kv(pos0, 6)
+        st.prefill(prompt, pos0)
+        out.append(st.logits())
+        st.free()
+    assert np.isfinite(out[0]).all() and np.array_equal(out[0], out[1])
+    w.free()
+
+
 def test_prefill_config2_shapes_match_oracle():
     """BASELINE config 2's model (Qwen2.5-0.5B INT8, tied lm_head) with 3 of
     the 24 layers, a 300-token synthetic prompt, against the oracle token by
