@@ -190,6 +190,22 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t rsrc_or_null(const void* base,
 }
 constexpr int kCacheNT = 2;   // buffer load cache policy: non-temporal (streamed once)
 
+// 1 KB of global memory (16 bytes per lane) into LDS at byte `lds`, past the
+// registers: at src + voff with a wave-uniform src, or at the lane's src.
+// The compiler does not count the request: wait_vm does.
+__device__ __forceinline__ void lds_load_1k(uint32_t lds, uint32_t voff, const char* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(src) : "memory");
+}
+__device__ __forceinline__ void lds_load_1k(uint32_t lds, const char* src) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+}
+// Until at most N vector memory requests of the wave are outstanding.
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+  static_assert(N < 64, "vmcnt range");
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+
 __device__ __forceinline__ u4_t load_u4_stream(const void* p) {
   return __builtin_nontemporal_load(reinterpret_cast<const u4_t*>(p));
 }

@@ -1002,6 +1002,8 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
     for (int l = 0; l < c.n_layers; ++l) {
       const LayerW& L = s->w->layers[l];
       const bool kv8 = s->kv_dtype != CQ_KV_FP16;
+      // E4M3 codes are coarse: prompts over that cache keep the sums, and so the codes, that they have always had
+      const bool keep_tile = s->kv_dtype == CQ_KV_FP8;
       _Float16* kc = kv8 ? nullptr : (_Float16*)(s->kcache + (size_t)l * s->layer_kv_halves);
       _Float16* vc = kv8 ? nullptr : (_Float16*)(s->vcache + (size_t)l * s->layer_kv_halves);
       int8_t* kc8 = kv8 ? reinterpret_cast<int8_t*>(s->kcache) + (size_t)l * s->layer_kv_halves : nullptr;
@@ -1021,7 +1023,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       g.out = (_Float16*)s->pf_q; g.head_dim = c.head_dim; g.pos0 = pos0 + c0; g.max_seq = c.max_seq_len;
       g.inv_freq = s->rope_inv_freq; g.kcache = kc; g.vcache = vc;
       g.kcache8 = kc8; g.vcache8 = vc8; g.kscale = ksc; g.vscale = vsc; g.kv_fmt = s->kv_dtype;
-      g.part = s->pf_part; g.part_bytes = kPrefillPartBytes;
+      g.part = s->pf_part; g.part_bytes = kPrefillPartBytes; g.keep_tile = keep_tile;
       CQ_TRY(launch_pf_gemm(g, st));
       PfAttnArgs at;
       at.q = (const _Float16*)s->pf_q; at.kcache = kc; at.vcache = vc; at.out = (_Float16*)s->pf_ao;
@@ -1038,7 +1040,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       PfGemmArgs o;
       o.mode = GM_RESID; o.quant = c.quant_type; o.A = (const _Float16*)s->pf_ao; o.M = M; o.N = d; o.K = qd;
       o.W[0] = L.wo; o.S[0] = (const _Float16*)L.so; o.panels = true; o.rows[0] = d; o.out = (_Float16*)s->pf_x;
-      o.part = s->pf_part; o.part_bytes = kPrefillPartBytes;
+      o.part = s->pf_part; o.part_bytes = kPrefillPartBytes; o.keep_tile = keep_tile;
       o.norm_w = (const _Float16*)L.post_norm; o.norm_eps = c.norm_eps;
       o.norm_out = (_Float16*)s->pf_a; o.norm_inv = s->pf_inv;
       CQ_TRY(launch_pf_gemm(o, st));
@@ -1047,12 +1049,12 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       m1.M = M; m1.N = I; m1.K = d; m1.W[0] = L.wg; m1.W[1] = L.wu;
       m1.S[0] = (const _Float16*)L.sg; m1.S[1] = (const _Float16*)L.su; m1.rows[0] = I; m1.rows[1] = I;
       m1.out = (_Float16*)s->pf_inter;
-      m1.part = s->pf_part; m1.part_bytes = kPrefillPartBytes;
+      m1.part = s->pf_part; m1.part_bytes = kPrefillPartBytes; m1.keep_tile = keep_tile;
       CQ_TRY(launch_pf_gemm(m1, st));
       PfGemmArgs m2;
       m2.mode = GM_RESID; m2.quant = c.quant_type; m2.A = (const _Float16*)s->pf_inter; m2.M = M; m2.N = d; m2.K = I;
       m2.W[0] = L.wd; m2.S[0] = (const _Float16*)L.sd; m2.rows[0] = d; m2.out = (_Float16*)s->pf_x;
-      m2.part = s->pf_part; m2.part_bytes = kPrefillPartBytes;
+      m2.part = s->pf_part; m2.part_bytes = kPrefillPartBytes; m2.keep_tile = keep_tile;
       // the next layer's input norm (every layer after this one is still to run)
       m2.norm_w = (const _Float16*)s->w->layers[l + 1].in_norm; m2.norm_eps = c.norm_eps;
       m2.norm_out = (_Float16*)s->pf_a; m2.norm_inv = s->pf_inv;

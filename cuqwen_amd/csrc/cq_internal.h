@@ -157,6 +157,7 @@ struct PfGemmArgs {
   float* kscale = nullptr;   // [n_kv][max_seq] of this layer
   float* vscale = nullptr;
   int kv_fmt = CQ_KV_INT8;   // CQ_KV_INT8 / CQ_KV_FP8 codes
+  bool keep_tile = false;    // always the 128-token tile, split by its rule alone (launch_pf_gemm)
   bool panels = false;       // W[0] / S[0] in 128-column panels (wo_to_panels), not row-major
   // RESID only, optional: RMSNorm of the updated rows (as launch_pf_norm) into
   // norm_out / norm_inv with weight norm_w

@@ -63,19 +63,6 @@ __device__ __forceinline__ float col_max(float v) {
   return fmaxf(__builtin_bit_cast(float, b[0]), __builtin_bit_cast(float, b[1]));
 }
 
-// 1 KB of global memory (16 bytes per lane at src + voff) into LDS at `lds`,
-// past the registers.  The compiler does not count the request: wait_vm does.
-__device__ __forceinline__ void lds_load_1k(uint32_t lds, uint32_t voff, const char* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(src) : "memory");
-}
-// Until at most N vector memory requests are outstanding (s_waitcnt's vmcnt
-// is in bits [3:0] and [15:14]; the other counters are left at their maxima).
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-  static_assert(N < 64, "vmcnt range");
-  asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-
 __device__ __forceinline__ float max3(float a, float b, float c) {
   float d;
   asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));

@@ -579,22 +579,272 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(const PfGemmArgs
   }
 }
 
+// --------------------------------------------------- few tokens: weight stream
+// The GEMM of a short prompt (or of a small matrix).  A block is TT slices of
+// 16 tokens by 128 weight rows: 4 row groups of 32 rows times 2 K groups (each
+// takes one half of the block's K steps [kb, ke)), whose sums meet in LDS.  A
+// ninth wave streams the activations straight into LDS, NST - 1 stages ahead:
+// loads complete in issue order per wave, so a wave that requested both would
+// wait for weights of later steps whenever it needs activations.
+// What bounds it: each wave's step (unpack, LDS reads, matrix instructions,
+// a barrier) and the weight bytes about equally.  7B int4 gate/up at 27
+// tokens 34.6 us = 2.0 TB/s; with the weight loads alone 20, with everything
+// but them 21-25.  The 128-token tile it replaces there does the work of 128
+// tokens: 69 us as it was split, 54 unsplit; down 43 -> 22, QKV 18 -> 13, O
+// 16 -> 11 (with their epilogues).  0.5B int4 at 27 tokens: gate/up 37 -> 7.
+// Measured on the way: four scales per load instead of one 28 -> 22 us (8
+// tokens), K halves in one block instead of a second partial 43 -> 35.
+// FORM PS_ROWS / PS_PANELS: rows of the concatenated matrices (q | k | v, gate
+// | up), row-major or in 128-column panels; the fp32 sums are a partial that
+// the split epilogue finishes.  PS_SWIGLU: 16 gate and the same 16 up rows per
+// wave over the whole K, finished here.
+enum { PS_ROWS, PS_PANELS, PS_SWIGLU };
+constexpr int kPsRG = 4, kPsKG = 2;
+constexpr int kPsWaves = kPsRG * kPsKG, kPsThreads = (kPsWaves + 1) * kWave;
+constexpr int kPsRows = kPsRG * 32;
+constexpr int kPsUnroll = 4;   // steps per loop iteration: scales are fetched four groups at a time
+template <int Q, int TT> struct PsShape {
+  static constexpr int D = Q == CQ_QUANT_INT4 ? 4 : 2;   // weight steps in flight
+  static constexpr int NST = TT == 4 ? 3 : 4;            // stages
+  static constexpr int XT = 16 * TT * kPfK;              // halves of one step's activations
+  static constexpr int XS = kPsKG * XT;                  // a stage: one step of each K group
+  static constexpr int OCC = TT == 4 ? 3 : 5;            // waves per SIMD (5: two blocks on a CU)
+};
+struct __attribute__((packed, aligned(2))) PsScales { uint64_t v; };   // four consecutive fp16 scales of a row
+
+template <int Q, int FORM, int TT>
+__global__ __launch_bounds__(kPsThreads, (PsShape<Q, TT>::OCC)) void pf_stream_kernel(const PfGemmArgs a) {
+  using SH = PsShape<Q, TT>;
+  constexpr int RT = 2, L = PfW<Q>::LOADS, D = SH::D, NST = SH::NST, XT = SH::XT, XS = SH::XS, U = kPsUnroll;
+  static_assert(U % D == 0, "register sets keep fixed indices");
+  __shared__ __align__(16) _Float16 xs[NST * XS];
+  const int lane = threadIdx.x & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int r = lane & 15, j = lane >> 4;
+  int rb, tb;
+  pf_block_tile((a.M + 16 * TT - 1) / (16 * TT), &rb, &tb);
+  const int m0 = tb * 16 * TT;
+  const int K = a.K, nks = K / kPfK;
+  const int kb = (int)((int64_t)blockIdx.z * nks / gridDim.z), ke = (int)((int64_t)(blockIdx.z + 1) * nks / gridDim.z);
+  const int n_st = (ke - kb + 1) / 2;   // K group 0 takes [kb, kb + n_st), K group 1 the rest
+
+  if (wave == kPsWaves) {
+    // 1 KB pieces of 4 token rows of one step, swizzled like the large tile's
+    // (pf_slot); steps past the range repeat the last
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)xs;
+    const char* row[4 * TT];
+#pragma unroll
+    for (int q = 0; q < 4 * TT; ++q) {
+      const int t = 4 * q + (lane >> 4);
+      row[q] = reinterpret_cast<const char*>(a.A + (int64_t)min(m0 + t, a.M - 1) * K + pf_slot(t, lane & 15) * 8);
+    }
+    auto request = [&](int st) {
+#pragma unroll
+      for (int kg = 0; kg < kPsKG; ++kg)
+#pragma unroll
+        for (int q = 0; q < 4 * TT; ++q)
+          lds_load_1k(lds0 + ((st % NST) * XS + kg * XT + q * 512) * 2, row[q] + min(kb + kg * n_st + st, ke - 1) * (kPfK * 2));
+    };
+#pragma unroll
+    for (int st = 0; st < NST - 1; ++st) request(st);
+    for (int st = 0; st < n_st; ++st) {
+      wait_vm<(NST - 2) * kPsKG * 4 * TT>();   // stage st is there
+      lds_barrier();
+      request(st + NST - 1);   // into the slot of stage st - 1, read before this barrier
+    }
+    wait_vm<0>();   // nothing may land once the stages are reused
+    __syncthreads();
+    __syncthreads();
+    if constexpr (FORM == PS_SWIGLU) __syncthreads();
+    return;
+  }
+
+  const int rg = wave % kPsRG, kg = wave / kPsRG;
+  const int k0 = kb + kg * n_st, n_k = min(n_st, ke - k0);   // the wave's steps
+  const int nt = FORM == PS_SWIGLU ? a.N : a.rows[0] + a.rows[1] + a.rows[2];
+  const int nw0 = FORM == PS_SWIGLU ? rb * (kPsRows / 2) + rg * 16 : rb * kPsRows + rg * 32;   // first row of the wave
+  const char* rowp[RT];
+  const _Float16* srow[RT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt) {
+    int local, mat;
+    if constexpr (FORM == PS_SWIGLU) {
+      mat = rt;
+      local = min(nw0 + r, nt - 1);
+    } else {
+      mat = pf_mat(a, min(nw0 + rt * 16 + r, nt - 1), &local);
+    }
+    const int64_t rbytes = FORM == PS_PANELS ? 64 * L : Q == CQ_QUANT_INT4 ? K / 2 : Q == CQ_QUANT_INT8 ? K : 2 * K;
+    rowp[rt] = reinterpret_cast<const char*>(sel3(a.W, mat)) + (int64_t)local * rbytes;
+    srow[rt] = Q == CQ_QUANT_FP16 ? nullptr : sel3(a.S, mat) + (FORM == PS_PANELS ? (int64_t)local : (int64_t)local * nks);
+  }
+  u4_t wv[D][RT][L];
+  auto w_load = [&](int i, int set) {   // the wave's step i (past the range: the block's last)
+    const int k = max(min(k0 + i, ke - 1), 0);
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const char* p = rowp[rt] + (int64_t)k * (FORM == PS_PANELS ? (int64_t)a.N * (64 * L) : 64 * L) + j * (L * 16);
+#pragma unroll
+      for (int l = 0; l < L; ++l) wv[set][rt][l] = load_u4(p + l * 16);
+    }
+  };
+  // scales of steps i .. i + 3, 16 bits each; a row-major row holds at least
+  // four (host), its last four are fetched where fewer follow
+  uint64_t sv[2][RT];
+  auto s_load = [&](int i, int set) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      if constexpr (FORM == PS_PANELS) {
+        uint64_t v = 0;
+#pragma unroll
+        for (int e = 0; e < U; ++e)
+          v |= (uint64_t)__builtin_bit_cast(uint16_t, srow[rt][(int64_t)min(k0 + i + e, ke - 1) * a.N]) << (16 * e);
+        sv[set][rt] = v;
+      } else {
+        const int k = k0 + i, k4 = max(min(k, nks - 4), 0);
+        sv[set][rt] = reinterpret_cast<const PsScales*>(srow[rt] + k4)->v >> (16 * min(k - k4, 3));
+      }
+    }
+  };
+  f4_t acc[RT][TT];
+#pragma unroll
+  for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+    for (int tt = 0; tt < TT; ++tt) acc[rt][tt] = f4_t{0.f, 0.f, 0.f, 0.f};
+  const UnpackRegs uk = unpack_regs();
+  if constexpr (Q != CQ_QUANT_FP16) s_load(0, 0);
+#pragma unroll
+  for (int d = 0; d < D; ++d) w_load(d, d);
+  for (int i0 = 0; i0 < n_st; i0 += U) {
+    if constexpr (Q != CQ_QUANT_FP16) s_load(i0 + U, 1);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int i = i0 + u;
+      if (u && i >= n_st) break;
+      __builtin_amdgcn_s_waitcnt(0xC07F);   // lgkmcnt(0): the stage before this one has been read
+      lds_barrier();
+      if (i < n_k) {
+        const _Float16* xb0 = xs + (i % NST) * XS + kg * XT;
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) {
+          h8_t xb[TT];
+#pragma unroll
+          for (int tt = 0; tt < TT; ++tt)
+            xb[tt] = *reinterpret_cast<const h8_t*>(&xb0[(tt * 16 + r) * kPfK + pf_slot(r, 4 * j + s4) * 8]);
+#pragma unroll
+          for (int rt = 0; rt < RT; ++rt) {
+            h8_t w = pf_unpack<Q>(wv[u % D][rt], s4, uk.m_lo, uk.m_hi, uk.magic);
+            if constexpr (Q != CQ_QUANT_FP16) {
+              const _Float16 sc = __builtin_bit_cast(_Float16, (uint16_t)(sv[0][rt] >> (16 * u)));
+              const h2_t s2 = {sc, sc};
+              u4_t uu = __builtin_bit_cast(u4_t, w);
+              uu.x = as_u32(as_h2(uu.x) * s2);
+              uu.y = as_u32(as_h2(uu.y) * s2);
+              uu.z = as_u32(as_h2(uu.z) * s2);
+              uu.w = as_u32(as_h2(uu.w) * s2);
+              w = __builtin_bit_cast(h8_t, uu);
+            }
+#pragma unroll
+            for (int tt = 0; tt < TT; ++tt)
+              acc[rt][tt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(w, xb[tt], acc[rt][tt], 0, 0, 0);
+          }
+        }
+      }
+      w_load(i + D, u % D);
+    }
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) sv[0][rt] = sv[1][rt];
+  }
+  // K group 1's sums into group 0's, over the stages
+  __syncthreads();
+  f4_t* red = reinterpret_cast<f4_t*>(xs) + rg * kWave * RT * TT + lane;
+  static_assert(kPsRG * kWave * 2 * TT * 16 <= NST * XS * 2, "sums fit");
+  if (kg == 1) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) red[(rt * TT + tt) * kWave] = acc[rt][tt];
+  }
+  __syncthreads();
+  if (kg == 0) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt)
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) acc[rt][tt] += red[(rt * TT + tt) * kWave];
+  }
+  if constexpr (FORM == PS_SWIGLU) {
+    // [token][64 rows] through LDS behind the sums, out in 8-element groups
+    constexpr int OS = kPsRows / 2 + 8;
+    static_assert(kPsRG * kWave * 2 * TT * 16 + 16 * TT * OS * 2 <= NST * XS * 2, "output tile fits");
+    _Float16* ot = xs + kPsRG * kWave * RT * TT * 8;
+    if (kg == 0) {
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        const float s = a.inv[min(m0 + tt * 16 + r, a.M - 1)];
+        h4_t o;
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          const float g = acc[0][tt][v] * s, u = acc[1][tt][v] * s;
+          o[v] = (_Float16)((g * (1.f / (1.f + expf(-g)))) * u);
+        }
+        *reinterpret_cast<h4_t*>(ot + (tt * 16 + r) * OS + rg * 16 + 4 * j) = o;
+      }
+    }
+    __syncthreads();
+    for (int idx = threadIdx.x; idx < 16 * TT * (kPsRows / 16); idx += kPsWaves * kWave) {
+      const int ml = idx / (kPsRows / 16), c = idx % (kPsRows / 16);
+      const int m = m0 + ml, n = rb * (kPsRows / 2) + 8 * c;
+      if (m < a.M && n < a.N)
+        *reinterpret_cast<h8_t*>(a.out + (int64_t)m * a.N + n) =
+            pf_group(*reinterpret_cast<const h8_t*>(ot + ml * OS + 8 * c), Q == CQ_QUANT_INT4);
+    }
+  } else if (kg == 0) {
+#pragma unroll
+    for (int rt = 0; rt < RT; ++rt) {
+      const int n = nw0 + rt * 16 + 4 * j;   // four rows of one matrix (their counts are multiples of 16)
+      if (n >= nt) continue;
+      int local;
+      const int mat = pf_mat(a, n, &local);
+#pragma unroll
+      for (int tt = 0; tt < TT; ++tt) {
+        const int m = m0 + tt * 16 + r;
+        if (m >= a.M) continue;
+        float* p = a.mode == GM_SWIGLU ? a.part + (((int64_t)blockIdx.z * 2 + mat) * a.M + m) * a.N + local
+                                       : a.part + ((int64_t)blockIdx.z * a.M + m) * a.N + n;
+        *reinterpret_cast<f4_t*>(p) = acc[rt][tt];
+      }
+    }
+  }
+}
+
 // Split-K epilogue of the SwiGLU GEMM: sums the S partials of each output
-// and applies the fused epilogue's arithmetic.
+// and applies the fused epilogue's arithmetic, one 8-element group (the
+// layout's unit) per thread.
 __global__ __launch_bounds__(256) void pf_split_swiglu(const PfGemmArgs a, int S) {
   const int64_t MN = (int64_t)a.M * a.N;
-  auto sum = [&](int mt, int64_t i) {
-    float v = 0.f;
-    for (int z = 0; z < S; ++z) v += a.part[((int64_t)z * 2 + mt) * MN + i];
-    return v;
-  };
-  for (int64_t idx = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; idx < MN; idx += (int64_t)gridDim.x * blockDim.x) {
-    const int m = (int)(idx / a.N), n = (int)(idx % a.N);
-    const float g = sum(0, idx) * a.inv[m], u = sum(1, idx) * a.inv[m];
+  const int64_t i = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 8;   // N is a multiple of 8
+  if (i >= MN) return;
+  const float inv = a.inv[i / a.N];
+  float v[2][8] = {};
+#pragma unroll 4
+  for (int z = 0; z < S; ++z)
+#pragma unroll
+    for (int mt = 0; mt < 2; ++mt) {
+      const f4_t* p = reinterpret_cast<const f4_t*>(a.part + ((int64_t)z * 2 + mt) * MN + i);
+      const f4_t p0 = p[0], p1 = p[1];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        v[mt][e] += p0[e];
+        v[mt][4 + e] += p1[e];
+      }
+    }
+  h8_t o;
+#pragma unroll
+  for (int e = 0; e < 8; ++e) {
+    const float g = v[0][e] * inv, u = v[1][e] * inv;
     const float sig = 1.f / (1.f + expf(-g));
-    a.out[(int64_t)m * a.N + pf_pos(n, a.quant == CQ_QUANT_INT4)] =
-        pf_val((float)(_Float16)((g * sig) * u), n, a.quant == CQ_QUANT_INT4);
+    o[e] = (_Float16)((g * sig) * u);
   }
+  *reinterpret_cast<h8_t*>(a.out + i) = pf_group(o, a.quant == CQ_QUANT_INT4);
 }
 
 // Split-K epilogue of a residual GEMM, one block per token row (N a
@@ -762,18 +1012,80 @@ int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __ha
   return CQ_OK;
 }
 
+// Sums S fp32 partials and finishes the GEMM.
+template <int MODE>
+static int launch_pf_split(const PfGemmArgs& a, int S, hipStream_t stream) {
+  if constexpr (MODE == GM_QKV) {
+    const int np_store = (a.kcache8 ? a.rows[0] : a.N) / 2, waves = kPfQkvThreads / kWave;
+    const int ny = (np_store / 4 + kPfQkvThreads - 1) / kPfQkvThreads +
+                   (a.kcache8 ? (2 * (a.rows[1] / a.head_dim) + waves - 1) / waves : 0);
+    if (a.head_dim == 128) hipLaunchKernelGGL((pf_split_qkv<128>), dim3(a.M, ny), dim3(kPfQkvThreads), 0, stream, a, S);
+    else hipLaunchKernelGGL((pf_split_qkv<64>), dim3(a.M, ny), dim3(kPfQkvThreads), 0, stream, a, S);
+  } else if constexpr (MODE == GM_RESID) {
+    hipLaunchKernelGGL(pf_split_resid, dim3(a.M), dim3(kPfResidThreads), 0, stream, a, S);
+  } else {
+    const int64_t groups = (int64_t)a.M * a.N / 8;
+    hipLaunchKernelGGL(pf_split_swiglu, dim3((unsigned)((groups + 255) / 256)), dim3(256), 0, stream, a, S);
+  }
+  CQ_HIP(hipGetLastError());
+  return CQ_OK;
+}
+
+// The weight stream with TT token slices, K split S ways (0: PS_SWIGLU).
+template <int Q, int MODE, int TT>
+static int launch_pf_stream(const PfGemmArgs& a, int S, hipStream_t stream) {
+  const int n_tb = (a.M + 16 * TT - 1) / (16 * TT);
+  if (MODE == GM_SWIGLU && S == 0) {
+    const int gx = ((a.N + kPsRows / 2 - 1) / (kPsRows / 2)) * n_tb;
+    hipLaunchKernelGGL((pf_stream_kernel<Q, PS_SWIGLU, TT>), dim3(gx), dim3(kPsThreads), 0, stream, a);
+    CQ_HIP(hipGetLastError());
+    return CQ_OK;
+  }
+  const int gx = ((a.rows[0] + a.rows[1] + a.rows[2] + kPsRows - 1) / kPsRows) * n_tb;
+  if (MODE == GM_RESID && a.panels)
+    hipLaunchKernelGGL((pf_stream_kernel<Q, PS_PANELS, TT>), dim3(gx, 1, S), dim3(kPsThreads), 0, stream, a);
+  else
+    hipLaunchKernelGGL((pf_stream_kernel<Q, PS_ROWS, TT>), dim3(gx, 1, S), dim3(kPsThreads), 0, stream, a);
+  CQ_HIP(hipGetLastError());
+  return launch_pf_split<MODE>(a, S, stream);
+}
+
+// The 128-token tile, split S ways over K (1: its fused epilogue).
 template <int Q, int MODE>
-static int launch_pf_gemm_m(const PfGemmArgs& a, hipStream_t stream) {
+static int launch_pf_tile(const PfGemmArgs& a, int S, hipStream_t stream) {
+  const int bn = PfShape<Q, MODE>::BN;
+  const int gx = ((a.N + bn - 1) / bn) * ((a.M + kPfTok - 1) / kPfTok);   // row blocks x token blocks
+  if (S > 1) {
+    hipLaunchKernelGGL((pf_gemm_kernel<Q, MODE, true>), dim3(gx, 1, S), dim3(kPfThreads), 0, stream, a);
+    CQ_HIP(hipGetLastError());
+    return launch_pf_split<MODE>(a, S, stream);
+  }
+  hipLaunchKernelGGL((pf_gemm_kernel<Q, MODE, false>), dim3(gx), dim3(kPfThreads), 0, stream, a);
+  CQ_HIP(hipGetLastError());
+  if (MODE == GM_RESID && a.norm_w) {
+    hipLaunchKernelGGL(pf_norm_rows, dim3(a.M), dim3(256), 0, stream, (const _Float16*)a.out, a.norm_w, a.norm_eps,
+                       a.N, a.norm_out, a.norm_inv, Q == CQ_QUANT_INT4);
+    CQ_HIP(hipGetLastError());
+  }
+  return CQ_OK;
+}
+
+// How a GEMM runs: the weight stream with tt token slices (split ways over K,
+// 0: PS_SWIGLU), or, tt = 0, the 128-token tile (split ways, 1: unsplit).
+struct PfPlan { int tt, split; };
+
+// The tile's split for more than 256 tokens.  Model: one block fits a CU (its
+// LDS), so B blocks take ceil(B / CUs) rounds and S splits ceil(S B / CUs)
+// rounds of 1/S the work; a full-K block runs at ~4.2 TFLOP/s per CU
+// (measured: int4 gate/up, 56 us per round of 256 blocks at K = 3584); the
+// split epilogue reads the S fp32 partials at ~2.8 TB/s after a launch of ~2
+// us (measured: QKV's 3 x 18.9 MB in 20.4 us, the residual's 2 x 14.7 MB in
+// 10.7 us).  Within the workspace.
+template <int Q, int MODE>
+static int pf_tile_split(const PfGemmArgs& a) {
   const int bn = PfShape<Q, MODE>::BN;
   const int gx = ((a.N + bn - 1) / bn) * ((a.M + kPfTok - 1) / kPfTok);   // row blocks x token blocks
   const int nks = a.K / kPfK, nmat = MODE == GM_SWIGLU ? 2 : 1;
-  // Split K when it shortens the GEMM plus its split epilogue.  Model: one
-  // block fits a CU (its LDS), so B blocks take ceil(B / CUs) rounds and S
-  // splits ceil(S B / CUs) rounds of 1/S the work; a full-K block runs at
-  // ~4.2 TFLOP/s per CU (measured: int4 gate/up, 56 us per round of 256
-  // blocks at K = 3584); the split epilogue reads the S fp32 partials at
-  // ~2.8 TB/s after a launch of ~2 us (measured: QKV's 3 x 18.9 MB in 20.4
-  // us, the residual's 2 x 14.7 MB in 10.7 us).  Within the workspace.
   int S = 1;
   if (a.part) {
     auto rounds = [&](int s) { return (double)(((int64_t)gx * s + kNumCUs - 1) / kNumCUs); };
@@ -790,31 +1102,72 @@ static int launch_pf_gemm_m(const PfGemmArgs& a, hipStream_t stream) {
       if (t < best) { best = t; S = s; }
     }
   }
-  if (S > 1) {
-    hipLaunchKernelGGL((pf_gemm_kernel<Q, MODE, true>), dim3(gx, 1, S), dim3(kPfThreads), 0, stream, a);
-    CQ_HIP(hipGetLastError());
-    if constexpr (MODE == GM_QKV) {
-      const int np_store = (a.kcache8 ? a.rows[0] : a.N) / 2, waves = kPfQkvThreads / kWave;
-      const int ny = (np_store / 4 + kPfQkvThreads - 1) / kPfQkvThreads +
-                     (a.kcache8 ? (2 * (a.rows[1] / a.head_dim) + waves - 1) / waves : 0);
-      if (a.head_dim == 128) hipLaunchKernelGGL((pf_split_qkv<128>), dim3(a.M, ny), dim3(kPfQkvThreads), 0, stream, a, S);
-      else hipLaunchKernelGGL((pf_split_qkv<64>), dim3(a.M, ny), dim3(kPfQkvThreads), 0, stream, a, S);
-    } else if constexpr (MODE == GM_RESID) {
-      hipLaunchKernelGGL(pf_split_resid, dim3(a.M), dim3(kPfResidThreads), 0, stream, a, S);
-    } else {
-      const int eb = (int)std::min<int64_t>(((int64_t)a.M * a.N + 255) / 256, 4096);
-      hipLaunchKernelGGL(pf_split_swiglu, dim3(eb), dim3(256), 0, stream, a, S);
-    }
-  } else {
-    hipLaunchKernelGGL((pf_gemm_kernel<Q, MODE, false>), dim3(gx), dim3(kPfThreads), 0, stream, a);
-    if (MODE == GM_RESID && a.norm_w) {
-      CQ_HIP(hipGetLastError());
-      hipLaunchKernelGGL(pf_norm_rows, dim3(a.M), dim3(256), 0, stream, (const _Float16*)a.out, a.norm_w, a.norm_eps,
-                         a.N, a.norm_out, a.norm_inv, Q == CQ_QUANT_INT4);
-    }
+  return S;
+}
+
+// Microseconds of either form, fitted to 5,000 measured (model, precision,
+// GEMM, tokens 8 .. 777, form, split) points; rms error 15 %, and the picks
+// cost 2 % (stream) and 4 % (tile) over the best of each form on average.
+// Tile: rounds of one block per CU, each a fixed part and its K steps.
+// Stream: the K steps of a wave times the blocks on the fullest CU.  Both: a
+// launch and the partials' bytes (written and read) for a split epilogue.
+template <int Q, int MODE>
+static double pf_tile_us(const PfGemmArgs& a, int S) {
+  constexpr double kFixed = Q == CQ_QUANT_FP16 ? 11.5 : 9.5, kStep = Q == CQ_QUANT_INT4 ? 1.6 : Q == CQ_QUANT_INT8 ? 1.85 : 2.6;
+  const int bn = PfShape<Q, MODE>::BN, nmat = MODE == GM_SWIGLU ? 2 : 1, nks = a.K / kPfK;
+  const int64_t blocks = (int64_t)((a.N + bn - 1) / bn) * ((a.M + kPfTok - 1) / kPfTok) * S;
+  const double mb = (double)S * nmat * a.M * a.N * sizeof(float) / 1e6;
+  const double per_mb = a.M > 256 ? 0.42 : 0.6;   // larger partials stream better
+  return -2.0 + (double)((blocks + kNumCUs - 1) / kNumCUs) * (kFixed + (nks + S - 1) / S * kStep) +
+         (S > 1 ? 2.3 + per_mb * mb : MODE == GM_QKV ? 18.0 : 0.0);
+}
+template <int Q>
+static double pf_stream_us(const PfGemmArgs& a, int tt, int S) {
+  constexpr double kFixed = Q == CQ_QUANT_INT4 ? 5.0 : Q == CQ_QUANT_INT8 ? 6.3 : 7.8;
+  constexpr double kStep[3] = {Q == CQ_QUANT_INT4 ? 0.70 : Q == CQ_QUANT_INT8 ? 1.13 : 2.1,
+                               Q == CQ_QUANT_INT4 ? 0.87 : Q == CQ_QUANT_INT8 ? 1.2 : 2.27,
+                               Q == CQ_QUANT_INT4 ? 1.14 : Q == CQ_QUANT_INT8 ? 1.44 : 2.45};
+  constexpr double kRound = Q == CQ_QUANT_FP16 ? 3.8 : 2.1;
+  const int rows = a.rows[0] + a.rows[1] + a.rows[2], s = std::max(S, 1), nks = a.K / kPfK;
+  const int64_t blocks = (int64_t)((rows + kPsRows - 1) / kPsRows) * ((a.M + 16 * tt - 1) / (16 * tt)) * s;
+  const double per_cu = (double)((blocks + kNumCUs - 1) / kNumCUs), steps = ((nks + s - 1) / s + 1) / 2;
+  return kFixed + steps * kStep[tt / 2] * per_cu + kRound * (per_cu - 1) +
+         (S ? 3.5 + 0.57 * S * a.M * (double)rows * sizeof(float) / 1e6 : 0.0);
+}
+
+template <int Q, int MODE>
+static PfPlan pf_plan(const PfGemmArgs& a) {
+  const int nks = a.K / kPfK, nmat = MODE == GM_SWIGLU ? 2 : 1;
+  PfPlan best{0, pf_tile_split<Q, MODE>(a)};
+  // above 1024 tokens the tile is the faster form at every preset's shapes;
+  // the stream fetches four scales of a row at a time
+  if (a.keep_tile || !a.part || a.M > 1024 || nks < 4) return best;
+  auto fits = [&](int s) { return (size_t)s * nmat * a.M * a.N * sizeof(float) <= a.part_bytes; };
+  if (a.M <= 256) {
+    for (int s = 1; s <= std::min(kPfMaxSplit, nks) && (s == 1 || fits(s)); ++s)
+      if (s == 1 || pf_tile_us<Q, MODE>(a, s) < pf_tile_us<Q, MODE>(a, best.split)) best.split = s;
   }
-  CQ_HIP(hipGetLastError());
-  return CQ_OK;
+  // the stream has to win by some of the model's error (where it errs for the
+  // stream: 0.5B int4 gate/up at 1000 tokens 42 against 36 us, 7B int4 QKV at
+  // 1024 78 against 68)
+  const double margin = a.M <= 512 ? 0.97 : MODE == GM_SWIGLU ? 0.88 : 0.95;
+  double t = margin * pf_tile_us<Q, MODE>(a, best.split);
+  for (int tt = 1; tt <= 4; tt *= 2)
+    for (int s = MODE == GM_SWIGLU ? 0 : 1; s <= std::min(32, nks) && fits(s); ++s)
+      if (const double u = pf_stream_us<Q>(a, tt, s); u < t) {
+        t = u;
+        best = PfPlan{tt, s};
+      }
+  return best;
+}
+
+template <int Q, int MODE>
+static int launch_pf_gemm_m(const PfGemmArgs& a, hipStream_t stream) {
+  const PfPlan p = pf_plan<Q, MODE>(a);
+  if (p.tt == 1) return launch_pf_stream<Q, MODE, 1>(a, p.split, stream);
+  if (p.tt == 2) return launch_pf_stream<Q, MODE, 2>(a, p.split, stream);
+  if (p.tt == 4) return launch_pf_stream<Q, MODE, 4>(a, p.split, stream);
+  return launch_pf_tile<Q, MODE>(a, p.split, stream);
 }
 
 template <int Q>

@@ -185,6 +185,34 @@ def test_prefill_attention_edges_match_decode(heads, kv_heads, hd, n, pos0, kv):
     w.free()
 
 
+# tokens around the 16-token slices and the stream's 16 / 32 / 64-token tiles;
+# K of 5, 9 (odd numbers of 128-wide steps: unequal K groups, scales of a row's
+# end fetched with its last four), 8 and 22 steps, row counts that do not fill
+# a 128-row block
+@pytest.mark.parametrize("n", [2, 15, 16, 17, 33, 64, 65, 130])
+@pytest.mark.parametrize("shape", [(640, 1152, 10, 2, 64), (1024, 2816, 8, 4, 128)])
+@pytest.mark.parametrize("quant", [0, 1, 2])
+def test_prefill_few_tokens_match_decode(quant, shape, n):
+    d, inter, heads, kv_heads, hd = shape
+    cfg = tiny_config(quant, dim=d, intermediate_size=inter, n_heads=heads, n_kv_heads=kv_heads, head_dim=hd, n_layers=3)
+    w = cq.synth_weights(cfg, 41)
+    prompt = _prompt(cfg, n, 8)
+    for kv in (cq.KV_FP16, cq.KV_INT8):
+        st, ref = cq.State(cfg, w, kv_dtype=kv), cq.State(cfg, w, kv_dtype=kv)
+        st.prefill(prompt, 0)
+        for i, t in enumerate(prompt):
+            ref.forward(t, i, [])
+        assert _rel(st.logits(), ref.logits()) <= TOL
+        # an int8 row may differ by a code, 1/127 of its maximum
+        tol = TOL if kv == cq.KV_FP16 else 2e-2
+        for h in range(kv_heads):
+            for kind in (0, 1):
+                assert _rel(st.kv_read(2, h, kind, n), ref.kv_read(2, h, kind, n)) <= tol, (h, kind)
+        st.free()
+        ref.free()
+    w.free()
+
+
 @pytest.mark.parametrize("hd,n,pos0", [(64, 40, 0), (128, 3, 600), (128, 33, 5)])
 def test_prefill_ignores_stale_cache(hd, n, pos0):
     """Whatever the cache holds past the context (NaN here) stays out of the
