@@ -204,7 +204,8 @@ struct cq_state {
   char* pf_arena = nullptr;
   __half *pf_x = nullptr, *pf_a = nullptr, *pf_q = nullptr, *pf_ao = nullptr, *pf_inter = nullptr;
   float* pf_inv = nullptr;
-  float* pf_part = nullptr;   // split-K partials of the prefill GEMMs
+  float* pf_rope = nullptr;   // sines and cosines of the chunk's positions
+  float* pf_part = nullptr;   // split-K partials of the prefill GEMMs, key-range partials of its attention
   int* pf_tokens = nullptr;
   int* pf_tokens_host = nullptr;   // pinned staging of a chunk's ids
   hipEvent_t pf_copied = nullptr;  // the staging buffer's last upload has completed
@@ -923,7 +924,9 @@ extern "C" int cq_state_kv_write(cq_state* s, int32_t layer, int32_t kv_head, in
 namespace {
 
 constexpr int kPrefillChunk = 2048;   // tokens per pass through the layers
-constexpr size_t kPrefillPartBytes = 64u << 20;   // split-K partials (small chunks)
+// split-K and key-range partials; 128 MB takes the splits that pay at a full
+// pass (7B QKV 136 -> 125 us in 2 x 38 MB, 14B down 399 -> 350 in 3 x 42)
+constexpr size_t kPrefillPartBytes = 128u << 20;
 
 int prefill_workspace(cq_state* s) {
   if (s->pf_arena) return CQ_OK;
@@ -932,7 +935,8 @@ int prefill_workspace(cq_state* s) {
   size_t off = 0;
   auto take = [&](size_t bytes) { size_t o = off; off = align_up(off + bytes); return o; };
   const size_t o_x = take(C * d * 2), o_a = take(C * d * 2), o_q = take(C * qd * 2), o_ao = take(C * qd * 2),
-               o_i = take(C * I * 2), o_inv = take(C * 4), o_t = take(C * 4), o_p = take(kPrefillPartBytes);
+               o_i = take(C * I * 2), o_inv = take(C * 4), o_t = take(C * 4),
+               o_r = take(C * c.head_dim * 4), o_p = take(kPrefillPartBytes);
   // the three parts are committed to the state together, or not at all
   char* a = nullptr;
   int* staging = nullptr;
@@ -954,6 +958,7 @@ int prefill_workspace(cq_state* s) {
   s->pf_x = (__half*)(a + o_x); s->pf_a = (__half*)(a + o_a); s->pf_q = (__half*)(a + o_q);
   s->pf_ao = (__half*)(a + o_ao); s->pf_inter = (__half*)(a + o_i); s->pf_inv = (float*)(a + o_inv);
   s->pf_tokens = (int*)(a + o_t);
+  s->pf_rope = (float*)(a + o_r);
   s->pf_part = (float*)(a + o_p);
   return CQ_OK;
 }
@@ -998,7 +1003,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
     std::memcpy(s->pf_tokens_host, tokens + c0, (size_t)M * 4);
     CQ_HIP(hipMemcpyAsync(s->pf_tokens, s->pf_tokens_host, (size_t)M * 4, hipMemcpyHostToDevice, st));
     CQ_HIP(hipEventRecord(s->pf_copied, st));
-    CQ_TRY(launch_pf_embed(s->w->embed, s->pf_tokens, M, d, s->pf_x, st));
+    CQ_TRY(launch_pf_embed(s->w->embed, s->pf_tokens, M, d, s->pf_x, s->rope_inv_freq, c.head_dim, pos0 + c0, s->pf_rope, st));
     for (int l = 0; l < c.n_layers; ++l) {
       const LayerW& L = s->w->layers[l];
       const bool kv8 = s->kv_dtype != CQ_KV_FP16;
@@ -1021,7 +1026,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       g.bias[0] = (const _Float16*)L.bq; g.bias[1] = (const _Float16*)L.bk; g.bias[2] = (const _Float16*)L.bv;
       g.rows[0] = qd; g.rows[1] = kvd; g.rows[2] = kvd;
       g.out = (_Float16*)s->pf_q; g.head_dim = c.head_dim; g.pos0 = pos0 + c0; g.max_seq = c.max_seq_len;
-      g.inv_freq = s->rope_inv_freq; g.kcache = kc; g.vcache = vc;
+      g.rope = s->pf_rope; g.kcache = kc; g.vcache = vc;
       g.kcache8 = kc8; g.vcache8 = vc8; g.kscale = ksc; g.vscale = vsc; g.kv_fmt = s->kv_dtype;
       g.part = s->pf_part; g.part_bytes = kPrefillPartBytes; g.keep_tile = keep_tile;
       CQ_TRY(launch_pf_gemm(g, st));

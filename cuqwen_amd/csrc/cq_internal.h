@@ -145,7 +145,7 @@ struct PfGemmArgs {
   int rows[3] = {0, 0, 0};
   _Float16* out = nullptr;
   int head_dim = 0, pos0 = 0, max_seq = 0;
-  const double* inv_freq = nullptr;
+  const float* rope = nullptr;   // QKV: sines [M][head_dim / 2] of the positions, then the cosines (launch_pf_embed)
   _Float16* kcache = nullptr;
   _Float16* vcache = nullptr;
   // split-K workspace (fp32 partials); nullptr: no split
@@ -157,7 +157,7 @@ struct PfGemmArgs {
   float* kscale = nullptr;   // [n_kv][max_seq] of this layer
   float* vscale = nullptr;
   int kv_fmt = CQ_KV_INT8;   // CQ_KV_INT8 / CQ_KV_FP8 codes
-  bool keep_tile = false;    // always the 128-token tile, split by its rule alone (launch_pf_gemm)
+  bool keep_tile = false;    // always the 128-token tile, split by its rule alone (E4M3 cache: the codes stay the same)
   bool panels = false;       // W[0] / S[0] in 128-column panels (wo_to_panels), not row-major
   // RESID only, optional: RMSNorm of the updated rows (as launch_pf_norm) into
   // norm_out / norm_inv with weight norm_w
@@ -185,7 +185,9 @@ struct PfAttnArgs {
 };
 int launch_pf_norm(const __half* x, const __half* w, float eps, int M, int dim, __half* A, float* inv, int quant,
                    hipStream_t stream);
-int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __half* x, hipStream_t stream);
+// Embedding rows and the RoPE table of positions pos0 .. pos0 + M (`rope`: M * head_dim floats).
+int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __half* x, const double* inv_freq,
+                    int head_dim, int pos0, float* rope, hipStream_t stream);
 int launch_pf_row_natural(const __half* src, __half* dst, int n, int quant, hipStream_t stream);
 int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream);
 int launch_pf_attention(const PfAttnArgs& a, hipStream_t stream);

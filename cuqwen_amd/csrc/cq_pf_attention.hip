@@ -485,9 +485,12 @@ __global__ __launch_bounds__(kPaMergeThreads) void pf_attention_merge(const PfAt
 // coarse number (a step is up to 1/8 of the value), so one different rounding
 // anywhere in the layers before turns some of a prompt's codes into their
 // neighbours.  Prompts over this cache therefore keep this kernel (and the
-// GEMMs' 128-token tile, see launch_pf_gemm) and with them the codes that
+// GEMMs' 128-token tile, PfGemmArgs::keep_tile) and with them the codes that
 // they have always had, although the kernel above is the faster one (84 ->
-// 47 us with int8 codes at 777 tokens after 3000, 12 / 2 heads).
+// 47 us with int8 codes at 777 tokens after 3000, 12 / 2 heads).  (Bit for
+// bit where the QKV tile is split over K; passes of more than about 1000
+// tokens run it unsplit, and its rotation is contracted differently since
+// the sines come from a table: 3 in a million of a layer's K codes.)
 template <int HD>
 __global__ __launch_bounds__(kAttnThreads) void pf_attention_e4m3_kernel(const PfAttnArgs a) {
   constexpr int KK = HD / 32, DT = HD / 16;

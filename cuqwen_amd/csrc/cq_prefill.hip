@@ -37,6 +37,7 @@ constexpr int kPfWaves = 8;
 constexpr int kPfThreads = kPfWaves * 64;
 constexpr int kPfK = 128;         // K per main-loop step (one quantization group)
 constexpr int kPfMaxSplit = 8;
+constexpr size_t kPfKeptPart = 64u << 20;   // partials that keep_tile's split rule reckons with
 
 // ------------------------------------------------------------- row norm
 // RMSNorm of one token row by one block (dim a multiple of 8): A row =
@@ -76,11 +77,19 @@ __global__ __launch_bounds__(256) void pf_norm_rows(const _Float16* x, const _Fl
   pf_norm_row(x + (int64_t)m * dim, w, eps, dim, A + (int64_t)m * dim, inv + m, int4, red);
 }
 
-// Embedding rows of the chunk's tokens (kernels.cu:85-103).
-__global__ __launch_bounds__(256) void pf_embed(const u4_t* embed, const int* tokens, u4_t* x, int vec_dim) {
+// Embedding rows of the chunk's tokens (kernels.cu:85-103), and the RoPE
+// sines and cosines of their positions, [M][half] each: every layer's QKV
+// epilogue reads them (the angle is reduced in double: computed per pair they
+// were a third of the unsplit epilogue).
+__global__ __launch_bounds__(256) void pf_embed(const u4_t* embed, const int* tokens, u4_t* x, int vec_dim,
+                                                const double* inv_freq, int half, int pos0, float* rope) {
   const int m = blockIdx.x;
   const int64_t t = tokens[m];
   for (int i = threadIdx.x; i < vec_dim; i += blockDim.x) x[(int64_t)m * vec_dim + i] = embed[t * vec_dim + i];
+  if ((int)threadIdx.x < half) {
+    float* sn = rope + (int64_t)m * half + threadIdx.x;
+    rope_sincos(pos0 + m, inv_freq[threadIdx.x], sn, sn + (int64_t)gridDim.x * half);
+  }
 }
 
 // ------------------------------------------------------------------ GEMM
@@ -126,24 +135,35 @@ __device__ __forceinline__ int pf_mat(const PfGemmArgs& a, int row, int* local) 
   return 2;
 }
 
-// One rotated pair (rows local, local + hd/2 of matrix mat) of token m:
-// q into the Q buffer, k / v into the cache at position pos0 + m.
-__device__ __forceinline__ void pf_qkv_store(const PfGemmArgs& a, int mat, int local, int m, _Float16 h0, _Float16 h1) {
+// Four consecutive rotated pairs (rows local + e, local + hd/2 + e of matrix
+// mat, e < 4) of token m: q into the Q buffer, k / v into the fp16 cache at
+// position pos0 + m.
+__device__ __forceinline__ void pf_qkv_store4(const PfGemmArgs& a, int mat, int local, int m, h4_t h0, h4_t h1) {
   const int hd = a.head_dim, half = hd / 2;
   if (mat == 0) {
-    a.out[(int64_t)m * a.rows[0] + local] = h0;
-    a.out[(int64_t)m * a.rows[0] + local + half] = h1;
+    *reinterpret_cast<h4_t*>(a.out + (int64_t)m * a.rows[0] + local) = h0;
+    *reinterpret_cast<h4_t*>(a.out + (int64_t)m * a.rows[0] + local + half) = h1;
+    return;
+  }
+  const int kvh = local / hd, i = local % hd, pos = a.pos0 + m;
+  if (mat == 1) {   // four consecutive elements of a K row are contiguous in the tiled cache
+    *reinterpret_cast<h4_t*>(a.kcache + kv_k_offset(kvh, pos, i, a.max_seq, hd)) = h0;
+    *reinterpret_cast<h4_t*>(a.kcache + kv_k_offset(kvh, pos, i + half, a.max_seq, hd)) = h1;
   } else {
-    const int kvh = local / hd, i = local % hd, pos = a.pos0 + m;
-    _Float16* c = mat == 1 ? a.kcache : a.vcache;
-    if (mat == 1) {
-      c[kv_k_offset(kvh, pos, i, a.max_seq, hd)] = h0;
-      c[kv_k_offset(kvh, pos, i + half, a.max_seq, hd)] = h1;
-    } else {
-      c[kv_v_offset(kvh, pos, i, a.max_seq, hd)] = h0;
-      c[kv_v_offset(kvh, pos, i + half, a.max_seq, hd)] = h1;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      a.vcache[kv_v_offset(kvh, pos, i + e, a.max_seq, hd)] = h0[e];
+      a.vcache[kv_v_offset(kvh, pos, i + half + e, a.max_seq, hd)] = h1[e];
     }
   }
+}
+// RoPE of four consecutive pairs of token m (the table of pf_embed).
+__device__ __forceinline__ void pf_rope4(const PfGemmArgs& a, int m, int i, float* y0, float* y1) {
+  const int half = a.head_dim / 2;
+  const float* p = a.rope + (int64_t)m * half + i;
+  const f4_t sn = *reinterpret_cast<const f4_t*>(p), cs = *reinterpret_cast<const f4_t*>(p + (int64_t)a.M * half);
+#pragma unroll
+  for (int e = 0; e < 4; ++e) rope_apply(y0[e], y1[e], sn[e], cs[e]);
 }
 
 // One (token, kv head) row into the quantized cache: s = max|x| / code max
@@ -225,7 +245,7 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(const PfGemmArgs
   constexpr int NMAT = SH::NMAT, RT = SH::RT, WROWS = SH::WROWS, BN = SH::BN, TT = kPfTT;
   constexpr int L = PfW<Q>::LOADS;
   constexpr int XS = kPfTok * kPfK;                         // halves of one activation stage
-  constexpr int OT = MODE == GM_QKV ? kPfTok / 2 * (BN + 2) : 0;   // QKV epilogue tile (half the tokens x rows)
+  constexpr int OT = MODE == GM_QKV ? kPfTok / 2 * (BN + 4) : 0;   // QKV epilogue tile (half the tokens x rows)
   constexpr int NS = 2;                                     // LDS stages
   // the epilogues reuse the stages: QKV tile, residual fp32 half tile
   constexpr int SM = std::max({NS * XS, OT, kPfTok / 2 * (BN + 4) * 2});
@@ -517,10 +537,10 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(const PfGemmArgs
     // QKV: norm scale, bias, fp16 into LDS (over the activation buffers, all
     // reads of which finished at the loop's last barrier), 64 tokens per
     // pass, token-major rows; then pairs (i, i + hd/2) of each head rotate
-    // (q, k) and go to Q or the KV cache, consecutive threads taking
-    // consecutive pairs of one token (so Q's stores are contiguous)
+    // (q, k) and go to Q or the KV cache, four pairs per thread, consecutive
+    // threads taking consecutive pairs of one token (so Q's stores are contiguous)
     constexpr int HT = kPfTok / 2;
-    constexpr int LDQ = BN + 2;   // odd dword stride: the token-per-lane reads below are conflict-free
+    constexpr int LDQ = BN + 4;   // 8-byte rows for the four-pair reads
     static_assert(HT * LDQ <= SM, "QKV staging fits");
     _Float16* ot = smem;
     const int hd = a.head_dim, half = hd / 2;
@@ -542,25 +562,59 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(const PfGemmArgs
             ot[(ml - h * HT) * LDQ + nl] = (_Float16)y;   // q/k/v are fp16 before RoPE (kernels.cu:470)
           }
       __syncthreads();
-      for (int idx = threadIdx.x; idx < (BN / 2) * HT; idx += kPfThreads) {
-        const int pi = idx % (BN / 2), ml = idx / (BN / 2);   // pair pi of the block's BN/2 pairs
+      for (int idx = threadIdx.x; idx < (BN / 8) * HT; idx += kPfThreads) {
+        const int pi = 4 * (idx % (BN / 8)), ml = idx / (BN / 8);   // pairs pi .. pi + 3 of the block's BN/2
         const int nl0 = (pi / half) * hd + pi % half, nl1 = nl0 + half;
         const int n0 = nb0 + nl0, m = m0 + h * HT + ml;
         if (n0 >= a.N || m >= a.M) continue;
         int local;
         const int mat = pf_mat(a, n0, &local);
-        float y0 = (float)ot[ml * LDQ + nl0], y1 = (float)ot[ml * LDQ + nl1];
-        const int pos = a.pos0 + m, i = local % hd;
-        if (mat < 2) rope_rotate(y0, y1, pos, a.inv_freq[i]);
+        if (mat == 2) continue;   // not rotated: stored as they stand below
+        h4_t h0 = *reinterpret_cast<const h4_t*>(&ot[ml * LDQ + nl0]), h1 = *reinterpret_cast<const h4_t*>(&ot[ml * LDQ + nl1]);
+        float y0[4], y1[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          y0[e] = (float)h0[e];
+          y1[e] = (float)h1[e];
+        }
+        pf_rope4(a, m, local % hd, y0, y1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          h0[e] = (_Float16)y0[e];
+          h1[e] = (_Float16)y1[e];
+        }
         if (a.kcache8 && mat > 0) {
           // quantized cache: rotated values back into the tile, quantized per head below
-          ot[ml * LDQ + nl0] = (_Float16)y0;
-          ot[ml * LDQ + nl1] = (_Float16)y1;
+          *reinterpret_cast<h4_t*>(&ot[ml * LDQ + nl0]) = h0;
+          *reinterpret_cast<h4_t*>(&ot[ml * LDQ + nl1]) = h1;
         } else {
-          pf_qkv_store(a, mat, local, m, (_Float16)y0, (_Float16)y1);
+          pf_qkv_store4(a, mat, local, m, h0, h1);
         }
       }
-      if (a.kcache8) {
+      if (!a.kcache8) {
+        // V: the tiled cache keeps the four positions of an aligned group of
+        // four side by side, so a thread takes one dim of such a group (8
+        // bytes; one position at a time, 2 bytes to a line each, the two
+        // blocks of V rows took 20 us longer than the rest of the launch)
+        const int v0 = max(a.rows[0] + a.rows[1] - nb0, 0), nv = min(BN, a.N - nb0) - v0;
+        const int p0 = a.pos0 + m0 + h * HT, cnt = min(HT, a.M - m0 - h * HT);
+        const int g0 = p0 >> 2, ng = nv > 0 && cnt > 0 ? ((p0 + cnt - 1) >> 2) - g0 + 1 : 0;
+        for (int idx = threadIdx.x; idx < ng * nv; idx += kPfThreads) {
+          const int nl = v0 + idx % nv, pos = 4 * (g0 + idx / nv), ml = pos - p0;
+          const int local = nb0 + nl - a.rows[0] - a.rows[1];
+          _Float16* dst = a.vcache + kv_v_offset(local / hd, pos, local % hd, a.max_seq, hd);
+          h4_t v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = ot[min(max(ml + e, 0), HT - 1) * LDQ + nl];
+          if (ml >= 0 && ml + 3 < cnt) {
+            *reinterpret_cast<h4_t*>(dst) = v;
+          } else {
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+              if (ml + e >= 0 && ml + e < cnt) dst[e] = v[e];
+          }
+        }
+      } else {
         __syncthreads();
         const int heads = BN / hd;
         for (int idx = threadIdx.x; idx < heads * HT; idx += kPfThreads) {
@@ -816,6 +870,16 @@ __global__ __launch_bounds__(kPsThreads, (PsShape<Q, TT>::OCC)) void pf_stream_k
   }
 }
 
+// half(a * b) with the product rounded once (v_fma_mixlo_f16), whatever the
+// code around it: two conversions that the compiler packs into one
+// instruction round the product to 32 bits first, and a prompt's E4M3 codes
+// hang on that last bit.
+__device__ __forceinline__ _Float16 mul_to_half(float a, float b) {
+  _Float16 r = (_Float16)(a * b);
+  asm("" : "+v"(r));
+  return r;
+}
+
 // Split-K epilogue of the SwiGLU GEMM: sums the S partials of each output
 // and applies the fused epilogue's arithmetic, one 8-element group (the
 // layout's unit) per thread.
@@ -842,7 +906,7 @@ __global__ __launch_bounds__(256) void pf_split_swiglu(const PfGemmArgs a, int S
   for (int e = 0; e < 8; ++e) {
     const float g = v[0][e] * inv, u = v[1][e] * inv;
     const float sig = 1.f / (1.f + expf(-g));
-    o[e] = (_Float16)((g * sig) * u);
+    o[e] = mul_to_half(g * sig, u);
   }
   *reinterpret_cast<h8_t*>(a.out + i) = pf_group(o, a.quant == CQ_QUANT_INT4);
 }
@@ -881,19 +945,16 @@ __global__ __launch_bounds__(kPfResidThreads) void pf_split_resid(const PfGemmAr
 
 // Split-K epilogue of the QKV GEMM, blockIdx.x = token: sums the partials,
 // applies the norm scale and bias (q / k / v are fp16 before RoPE,
-// kernels.cu:470), rotates q and k with the token's sines and cosines
-// (computed once per block) and stores q, and k / v into the cache; block y
+// kernels.cu:470), rotates q and k with the token's sines and cosines and
+// stores q, and k / v into the cache; block y
 // takes pairs [1024 y, 1024 y + 1024), four per thread.  A quantized cache takes each (k or v,
 // kv head) row through one wave of the blocks past the pairs.
 constexpr int kPfQkvThreads = 256;
 template <int HD>
 __global__ __launch_bounds__(kPfQkvThreads) void pf_split_qkv(const PfGemmArgs a, int S) {
   constexpr int HALF = HD / 2;
-  __shared__ float sn[HALF], cs[HALF];
   const int m = blockIdx.x, pos = a.pos0 + m;
   const int64_t MN = (int64_t)a.M * a.N;
-  for (int i = threadIdx.x; i < HALF; i += blockDim.x) rope_sincos(pos, a.inv_freq[i], &sn[i], &cs[i]);
-  __syncthreads();
   const float inv = a.inv[m];
   const float* prow = a.part + (int64_t)m * a.N;
   // fp16 value of row n (bias added, before RoPE)
@@ -927,29 +988,15 @@ __global__ __launch_bounds__(kPfQkvThreads) void pf_split_qkv(const PfGemmArgs a
     for (int e = 0; e < 4; ++e) {
       y0[e] = (float)(_Float16)(s0[e] * inv + (b ? (float)b[local + e] : 0.f));
       y1[e] = (float)(_Float16)(s1[e] * inv + (b ? (float)b[local + HALF + e] : 0.f));
-      if (mat < 2) rope_apply(y0[e], y1[e], sn[i + e], cs[i + e]);
     }
+    if (mat < 2) pf_rope4(a, m, i, y0, y1);
     h4_t h0, h1;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
       h0[e] = (_Float16)y0[e];
       h1[e] = (_Float16)y1[e];
     }
-    if (mat == 0) {
-      *reinterpret_cast<h4_t*>(a.out + (int64_t)m * a.rows[0] + local) = h0;
-      *reinterpret_cast<h4_t*>(a.out + (int64_t)m * a.rows[0] + local + HALF) = h1;
-    } else if (mat == 1) {   // four consecutive elements of a K row are contiguous in the tiled cache
-      const int kvh = local / HD;
-      *reinterpret_cast<h4_t*>(a.kcache + kv_k_offset(kvh, pos, i, a.max_seq, HD)) = h0;
-      *reinterpret_cast<h4_t*>(a.kcache + kv_k_offset(kvh, pos, i + HALF, a.max_seq, HD)) = h1;
-    } else {
-      const int kvh = local / HD;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        a.vcache[kv_v_offset(kvh, pos, i + e, a.max_seq, HD)] = h0[e];
-        a.vcache[kv_v_offset(kvh, pos, i + HALF + e, a.max_seq, HD)] = h1[e];
-      }
-    }
+    pf_qkv_store4(a, mat, local, m, h0, h1);
   } else {
     constexpr int E = HD / kWave;   // consecutive elements per lane
     const int lane = threadIdx.x & (kWave - 1), n_kv = a.rows[1] / HD;
@@ -962,7 +1009,10 @@ __global__ __launch_bounds__(kPfQkvThreads) void pf_split_qkv(const PfGemmArgs a
       for (int e = 0; e < E; ++e) {
         const int d = lane * E + e, i = d % HALF;
         float y0 = raw(nb + i), y1 = raw(nb + i + HALF);
-        if (mat == 1) rope_apply(y0, y1, sn[i], cs[i]);
+        if (mat == 1) {
+          const float* p = a.rope + (int64_t)m * HALF + i;
+          rope_apply(y0, y1, p[0], p[(int64_t)a.M * HALF]);
+        }
         x[e] = (float)(_Float16)(d < HALF ? y0 : y1);
       }
       int8_t q[E];
@@ -1005,9 +1055,10 @@ int launch_pf_row_natural(const __half* src, __half* dst, int n, int quant, hipS
   return CQ_OK;
 }
 
-int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __half* x, hipStream_t stream) {
+int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __half* x, const double* inv_freq,
+                    int head_dim, int pos0, float* rope, hipStream_t stream) {
   hipLaunchKernelGGL(pf_embed, dim3(M), dim3(256), 0, stream, reinterpret_cast<const u4_t*>(embed), tokens,
-                     reinterpret_cast<u4_t*>(x), dim / 8);
+                     reinterpret_cast<u4_t*>(x), dim / 8, inv_freq, head_dim / 2, pos0, rope);
   CQ_HIP(hipGetLastError());
   return CQ_OK;
 }
@@ -1091,13 +1142,12 @@ static int pf_tile_split(const PfGemmArgs& a) {
     auto rounds = [&](int s) { return (double)(((int64_t)gx * s + kNumCUs - 1) / kNumCUs); };
     const double t1 = (double)bn * nmat * kPfTok * a.K * 2 / 4.2e6;     // us, one round of full-K blocks
     const double part_us = (double)nmat * a.M * a.N * sizeof(float) / 2.8e6;   // us per split of partials
-    // QKV's unsplit epilogue (RoPE through an LDS tile, scattered cache
-    // stores) costs about what the split epilogue's pass does (measured: at
-    // 1024 tokens the unsplit QKV launch took ~25 us longer than the 3-way
-    // split plus its epilogue)
+    // QKV's unsplit epilogue (RoPE through an LDS tile, cache stores) costs
+    // about what a split epilogue's pass does (measured: 7B at 1024 tokens 72
+    // us unsplit, 67 split 3 ways; at 1536 71 and 100)
     double best = rounds(1) * t1 + (MODE == GM_QKV ? part_us + 2.0 : 0.0);
     for (int s = 2; s <= std::min(kPfMaxSplit, nks); ++s) {
-      if ((size_t)s * nmat * a.M * a.N * sizeof(float) > a.part_bytes) break;
+      if ((size_t)s * nmat * a.M * a.N * sizeof(float) > (a.keep_tile ? std::min(a.part_bytes, kPfKeptPart) : a.part_bytes)) break;
       const double t = rounds(s) / s * t1 + s * part_us + 2.0;
       if (t < best) { best = t; S = s; }
     }
@@ -1187,7 +1237,7 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream) {
     return fail(CQ_EINVAL, "prefill gemm: residual rows must be a multiple of 8 wide; the norm needs its outputs");
   if (a.panels && a.mode != GM_RESID) return fail(CQ_EINVAL, "prefill gemm: paneled weights are a residual-mode option");
   if (a.mode == GM_QKV) {
-    if (!a.inv || !a.W[1] || !a.W[2] || !a.inv_freq) return fail(CQ_EINVAL, "prefill gemm: qkv operands");
+    if (!a.inv || !a.W[1] || !a.W[2] || !a.rope) return fail(CQ_EINVAL, "prefill gemm: qkv operands");
     if (a.kcache8 ? (!a.vcache8 || !a.kscale || !a.vscale) : (!a.kcache || !a.vcache))
       return fail(CQ_EINVAL, "prefill gemm: qkv cache pointers");
     if (PfShape<CQ_QUANT_FP16, GM_QKV>::BN % a.head_dim || a.rows[0] % a.head_dim || a.rows[1] % a.head_dim || a.rows[0] + a.rows[1] + a.rows[2] != a.N)

@@ -213,6 +213,32 @@ def test_prefill_few_tokens_match_decode(quant, shape, n):
     w.free()
 
 
+# the unsplit QKV epilogue (enough row and token blocks that a split does not
+# pay) stores V by aligned groups of four positions: ragged ends and starts
+@pytest.mark.parametrize("n,pos0", [(1025, 0), (1051, 3), (1027, 6)])
+def test_prefill_unsplit_qkv_cache_rows(n, pos0):
+    cfg = tiny_config(2, n_heads=56, n_kv_heads=8, head_dim=64, dim=512, max_seq_len=2048, n_layers=1)
+    w = cq.synth_weights(cfg, 17)
+    prompt = _prompt(cfg, n, 5)
+    st, ref = cq.State(cfg, w), cq.State(cfg, w)
+    if pos0:
+        st.fill_kv(pos0, 5)
+        ref.fill_kv(pos0, 5)
+    st.prefill(prompt, pos0)
+    for i in range(0, n, 63):   # layer 0's rows depend on their own token alone
+        ref.forward(prompt[i], pos0 + i, [])
+    ref.forward(prompt[-1], pos0 + n - 1, [])
+    rows = [pos0 + i for i in range(0, n, 63)] + [pos0 + n - 1]
+    for h in range(8):
+        for kind in (0, 1):
+            a, b = st.kv_read(0, h, kind, pos0 + n + 8), ref.kv_read(0, h, kind, pos0 + n + 8)
+            assert _rel(a[rows], b[rows]) <= TOL, (h, kind)
+            assert np.array_equal(a[:pos0], b[:pos0]) and not a[pos0 + n:].any()
+    st.free()
+    w.free()
+    ref.free()
+
+
 @pytest.mark.parametrize("hd,n,pos0", [(64, 40, 0), (128, 3, 600), (128, 33, 5)])
 def test_prefill_ignores_stale_cache(hd, n, pos0):
     """Whatever the cache holds past the context (NaN here) stays out of the
