@@ -112,10 +112,6 @@ extern "C" int cq_compute_logits(int32_t lm_quant, const void* x, const void* W,
   return launch_gemv(a, as_stream(stream));
 }
 
-namespace cq {
-int launch_epoch_bump(uint32_t* d_epoch, hipStream_t stream);
-}
-
 // Workspace: [epoch uint32, padded to 256 B][stamp uint32 x vocab]; zero it
 // once before the first call.
 extern "C" size_t cq_penalty_workspace_bytes(int32_t vocab) { return 256 + (size_t)(vocab > 0 ? vocab : 0) * 4; }
@@ -127,7 +123,6 @@ extern "C" int cq_apply_repetition_penalty(void* logits, const int32_t* d_histor
   uint32_t* epoch = (uint32_t*)workspace;
   uint32_t* stamp = (uint32_t*)((char*)workspace + 256);
   const hipStream_t st = as_stream(stream);
-  CQ_TRY(launch_epoch_bump(epoch, st));
   CQ_TRY(launch_stamp_history(stamp, d_history, d_history_len, vocab, epoch, st));
   return launch_penalty_apply((__half*)logits, stamp, epoch, vocab, penalty, st);
 }
