@@ -971,8 +971,7 @@ int prefill_tail(cq_state* s, int M) {
   const cq_config& c = s->cfg;
   hipStream_t st = s->stream;
   const int d = c.dim, qd = c.n_heads * c.head_dim;
-  CQ_HIP(hipMemcpyAsync(s->x, s->pf_x + (size_t)(M - 1) * d, (size_t)d * 2, hipMemcpyDeviceToDevice, st));
-  CQ_TRY(launch_pf_row_natural(s->pf_ao + (size_t)(M - 1) * qd, s->xb, qd, c.quant_type, st));
+  CQ_TRY(launch_pf_last_row(s->pf_ao + (size_t)(M - 1) * qd, s->xb, qd, c.quant_type, s->pf_x + (size_t)(M - 1) * d, s->x, d, st));
   GemvArgs m1, m2;
   layer_gemvs(s, c.n_layers - 1, nullptr, &m1, &m2);
   fused_mlp(s, &m1, &m2);
@@ -1003,7 +1002,8 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
     std::memcpy(s->pf_tokens_host, tokens + c0, (size_t)M * 4);
     CQ_HIP(hipMemcpyAsync(s->pf_tokens, s->pf_tokens_host, (size_t)M * 4, hipMemcpyHostToDevice, st));
     CQ_HIP(hipEventRecord(s->pf_copied, st));
-    CQ_TRY(launch_pf_embed(s->w->embed, s->pf_tokens, M, d, s->pf_x, s->rope_inv_freq, c.head_dim, pos0 + c0, s->pf_rope, st));
+    CQ_TRY(launch_pf_embed(s->w->embed, s->pf_tokens, M, d, s->pf_x, s->rope_inv_freq, c.head_dim, pos0 + c0, s->pf_rope,
+                           s->w->layers[0].in_norm, c.norm_eps, s->pf_a, s->pf_inv, c.quant_type, st));
     for (int l = 0; l < c.n_layers; ++l) {
       const LayerW& L = s->w->layers[l];
       const bool kv8 = s->kv_dtype != CQ_KV_FP16;
@@ -1016,8 +1016,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       const size_t ls = (size_t)l * c.n_kv_heads * c.max_seq_len;
       float* ksc = kv8 ? s->kscale + ls : nullptr;
       float* vsc = kv8 ? s->vscale + ls : nullptr;
-      // layer l > 0: the previous layer's down GEMM left this norm in pf_a / pf_inv
-      if (l == 0) CQ_TRY(launch_pf_norm(s->pf_x, L.in_norm, c.norm_eps, M, d, s->pf_a, s->pf_inv, c.quant_type, st));
+      // the input norm is in pf_a / pf_inv: from the embedding, or the previous layer's down GEMM
       PfGemmArgs g;
       g.mode = GM_QKV; g.quant = c.quant_type; g.A = (const _Float16*)s->pf_a; g.inv = s->pf_inv;
       g.M = M; g.N = qd + 2 * kvd; g.K = d;

@@ -159,7 +159,7 @@ struct PfGemmArgs {
   int kv_fmt = CQ_KV_INT8;   // CQ_KV_INT8 / CQ_KV_FP8 codes
   bool keep_tile = false;    // always the 128-token tile, split by its rule alone (E4M3 cache: the codes stay the same)
   bool panels = false;       // W[0] / S[0] in 128-column panels (wo_to_panels), not row-major
-  // RESID only, optional: RMSNorm of the updated rows (as launch_pf_norm) into
+  // RESID only, optional: RMSNorm of the updated rows (half(x * w) and the scale) into
   // norm_out / norm_inv with weight norm_w
   const _Float16* norm_w = nullptr;
   float norm_eps = 0.f;
@@ -183,12 +183,15 @@ struct PfAttnArgs {
   size_t part_bytes = 0;
   int n_rb = 0, splits = 1;   // set by the launcher: row blocks per kv head, key ranges
 };
-int launch_pf_norm(const __half* x, const __half* w, float eps, int M, int dim, __half* A, float* inv, int quant,
-                   hipStream_t stream);
-// Embedding rows and the RoPE table of positions pos0 .. pos0 + M (`rope`: M * head_dim floats).
+// Embedding rows, the RoPE table of positions pos0 .. pos0 + M (`rope`: M *
+// head_dim floats) and the first layer's input norm (norm_out in the layout of
+// `quant`, norm_inv).
 int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __half* x, const double* inv_freq,
-                    int head_dim, int pos0, float* rope, hipStream_t stream);
-int launch_pf_row_natural(const __half* src, __half* dst, int n, int quant, hipStream_t stream);
+                    int head_dim, int pos0, float* rope, const __half* norm_w, float eps, __half* norm_out,
+                    float* norm_inv, int quant, hipStream_t stream);
+// Attention row src (layout of `quant`) to dst in natural order, x to x_out.
+int launch_pf_last_row(const __half* src, __half* dst, int n, int quant, const __half* x, __half* x_out, int dim,
+                       hipStream_t stream);
 int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream);
 int launch_pf_attention(const PfAttnArgs& a, hipStream_t stream);
 

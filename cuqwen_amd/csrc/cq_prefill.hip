@@ -6,8 +6,8 @@
 // Per layer and chunk of M tokens:
 //   RMSNorm         x -> half(x * w) and rsqrt(mean(x^2) + eps) per token
 //                   (the decode GEMVs' fused RMSNorm, kernels.cu:689-751):
-//                   pf_norm_rows for layer 0, later in the epilogue of the
-//                   residual GEMM that produces x
+//                   with the embedding for layer 0, later in the epilogue of
+//                   the residual GEMM that produces x
 //   pf_gemm<QKV>    Q / K / V rows, bias, RoPE at each token's position, K / V
 //                   into the cache (kernels.cu:402-474, :370-398, :326-347)
 //   pf_attention    causal FlashDecoding over the cache (kernels.cu:105-288
@@ -77,19 +77,36 @@ __global__ __launch_bounds__(256) void pf_norm_rows(const _Float16* x, const _Fl
   pf_norm_row(x + (int64_t)m * dim, w, eps, dim, A + (int64_t)m * dim, inv + m, int4, red);
 }
 
-// Embedding rows of the chunk's tokens (kernels.cu:85-103), and the RoPE
-// sines and cosines of their positions, [M][half] each: every layer's QKV
-// epilogue reads them (the angle is reduced in double: computed per pair they
-// were a third of the unsplit epilogue).
-__global__ __launch_bounds__(256) void pf_embed(const u4_t* embed, const int* tokens, u4_t* x, int vec_dim,
-                                                const double* inv_freq, int half, int pos0, float* rope) {
-  const int m = blockIdx.x;
-  const int64_t t = tokens[m];
-  for (int i = threadIdx.x; i < vec_dim; i += blockDim.x) x[(int64_t)m * vec_dim + i] = embed[t * vec_dim + i];
-  if ((int)threadIdx.x < half) {
-    float* sn = rope + (int64_t)m * half + threadIdx.x;
-    rope_sincos(pos0 + m, inv_freq[threadIdx.x], sn, sn + (int64_t)gridDim.x * half);
+// Embedding rows of the chunk's tokens (kernels.cu:85-103), the first layer's
+// input norm of them, and the RoPE sines and cosines of their positions,
+// [M][half] each: every layer's QKV epilogue reads them (the angle is reduced
+// in double: computed per pair they were a third of the unsplit epilogue).
+struct PfEmbedArgs {
+  const u4_t* embed;
+  const int* tokens;
+  _Float16* x;
+  int dim;
+  const double* inv_freq;
+  int half, pos0;
+  float* rope;
+  const _Float16* norm_w;
+  float eps;
+  _Float16* norm_out;
+  float* norm_inv;
+  bool int4;
+};
+__global__ __launch_bounds__(256) void pf_embed(const PfEmbedArgs a) {
+  __shared__ float red[16];
+  const int m = blockIdx.x, vec_dim = a.dim / 8;
+  const int64_t t = a.tokens[m];
+  _Float16* xr = a.x + (int64_t)m * a.dim;
+  for (int i = threadIdx.x; i < vec_dim; i += blockDim.x) *reinterpret_cast<u4_t*>(xr + 8 * i) = a.embed[t * vec_dim + i];
+  if ((int)threadIdx.x < a.half) {
+    float* sn = a.rope + (int64_t)m * a.half + threadIdx.x;
+    rope_sincos(a.pos0 + m, a.inv_freq[threadIdx.x], sn, sn + (int64_t)gridDim.x * a.half);
   }
+  // reads back the groups this thread has just written
+  pf_norm_row(xr, a.norm_w, a.eps, a.dim, a.norm_out + (int64_t)m * a.dim, a.norm_inv + m, a.int4, red);
 }
 
 // ------------------------------------------------------------------ GEMM
@@ -1028,37 +1045,35 @@ __global__ __launch_bounds__(kPfQkvThreads) void pf_split_qkv(const PfGemmArgs a
   }
 }
 
-// One row of a GEMM input back to natural order (the int4 layout stores each
-// 8-group as [0,4,1,5,2,6,3,7] with the odd elements / 16; the scale is a
-// power of two, so the round trip is exact for odd elements of magnitude at
-// least 2^-10 -- smaller ones lost low bits to the subnormal range on the way
-// in).
-__global__ __launch_bounds__(256) void pf_row_natural(const _Float16* src, _Float16* dst, int n, bool int4) {
-  for (int k = threadIdx.x; k < n; k += blockDim.x)
-    dst[k] = (_Float16)((float)src[pf_pos(k, int4)] * ((int4 && (k & 1)) ? 16.0f : 1.0f));
+// The last token's rows for the decode kernels that finish it: its attention
+// output back to natural order (the int4 layout stores each 8-group as
+// [0,4,1,5,2,6,3,7] with the odd elements / 16; the scale is a power of two,
+// so the round trip is exact for odd elements of magnitude at least 2^-10 --
+// smaller ones lost low bits to the subnormal range on the way in), and its
+// residual.
+__global__ __launch_bounds__(256) void pf_last_row(const _Float16* src, _Float16* dst, int n, bool int4,
+                                                   const _Float16* x, _Float16* x_out, int dim) {
+  const int k = blockIdx.x * blockDim.x + threadIdx.x;
+  if (k < n) dst[k] = (_Float16)((float)src[pf_pos(k, int4)] * ((int4 && (k & 1)) ? 16.0f : 1.0f));
+  if (k < dim) x_out[k] = x[k];
 }
 
 // ------------------------------------------------------------------ host
-int launch_pf_norm(const __half* x, const __half* w, float eps, int M, int dim, __half* A, float* inv,
-                   int quant, hipStream_t stream) {
-  if (M <= 0 || dim <= 0 || dim % 8) return fail(CQ_EINVAL, "prefill norm: rows must be a multiple of 8 wide");
-  hipLaunchKernelGGL(pf_norm_rows, dim3(M), dim3(256), 0, stream, (const _Float16*)x, (const _Float16*)w, eps, dim,
-                     (_Float16*)A, inv, quant == CQ_QUANT_INT4);
-  CQ_HIP(hipGetLastError());
-  return CQ_OK;
-}
-
-int launch_pf_row_natural(const __half* src, __half* dst, int n, int quant, hipStream_t stream) {
-  hipLaunchKernelGGL(pf_row_natural, dim3(1), dim3(256), 0, stream, (const _Float16*)src, (_Float16*)dst, n,
-                     quant == CQ_QUANT_INT4);
+int launch_pf_last_row(const __half* src, __half* dst, int n, int quant, const __half* x, __half* x_out, int dim,
+                       hipStream_t stream) {
+  hipLaunchKernelGGL(pf_last_row, dim3((std::max(n, dim) + 255) / 256), dim3(256), 0, stream, (const _Float16*)src,
+                     (_Float16*)dst, n, quant == CQ_QUANT_INT4, (const _Float16*)x, (_Float16*)x_out, dim);
   CQ_HIP(hipGetLastError());
   return CQ_OK;
 }
 
 int launch_pf_embed(const __half* embed, const int* tokens, int M, int dim, __half* x, const double* inv_freq,
-                    int head_dim, int pos0, float* rope, hipStream_t stream) {
-  hipLaunchKernelGGL(pf_embed, dim3(M), dim3(256), 0, stream, reinterpret_cast<const u4_t*>(embed), tokens,
-                     reinterpret_cast<u4_t*>(x), dim / 8, inv_freq, head_dim / 2, pos0, rope);
+                    int head_dim, int pos0, float* rope, const __half* norm_w, float eps, __half* norm_out,
+                    float* norm_inv, int quant, hipStream_t stream) {
+  if (M <= 0 || dim <= 0 || dim % 8) return fail(CQ_EINVAL, "prefill norm: rows must be a multiple of 8 wide");
+  PfEmbedArgs a{reinterpret_cast<const u4_t*>(embed), tokens, (_Float16*)x, dim, inv_freq, head_dim / 2, pos0, rope,
+                (const _Float16*)norm_w, eps, (_Float16*)norm_out, norm_inv, quant == CQ_QUANT_INT4};
+  hipLaunchKernelGGL(pf_embed, dim3(M), dim3(256), 0, stream, a);
   CQ_HIP(hipGetLastError());
   return CQ_OK;
 }
