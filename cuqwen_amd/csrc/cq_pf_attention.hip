@@ -63,11 +63,11 @@ __device__ __forceinline__ float col_max(float v) {
   return fmaxf(__builtin_bit_cast(float, b[0]), __builtin_bit_cast(float, b[1]));
 }
 
-__device__ __forceinline__ float max3(float a, float b, float c) {
-  float d;
-  asm("v_max3_f32 %0, %1, %2, %3" : "=v"(d) : "v"(a), "v"(b), "v"(c));
-  return d;
-}
+// One v_max3_f32, and not written as asm: the operands are matrix results, and
+// the compiler adds the wait states that these ask for (and that a register
+// that a product has yet to write asks of its next writer) only in front of
+// instructions of its own.
+__device__ __forceinline__ float max3(float a, float b, float c) { return fmaxf(fmaxf(a, b), c); }
 
 template <int HD, int KV8, int KH, int TPW>   // KV8: 0 fp16 cache, CQ_KV_INT8 int8 codes
 __global__ __launch_bounds__(kPaThreads, 2) void pf_attention_kernel(const PfAttnArgs a) {
