@@ -194,10 +194,10 @@ constexpr int kCacheNT = 2;   // buffer load cache policy: non-temporal (streame
 // registers: at src + voff with a wave-uniform src, or at the lane's src.
 // The compiler does not count the request: wait_vm does.
 __device__ __forceinline__ void lds_load_1k(uint32_t lds, uint32_t voff, const char* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(src) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" ::"s"(lds), "v"(voff), "s"(src) : "memory", "m0");
 }
 __device__ __forceinline__ void lds_load_1k(uint32_t lds, const char* src) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(src) : "memory", "m0");
 }
 // Until at most N vector memory requests of the wave are outstanding.
 template <int N>

@@ -127,3 +127,16 @@ def test_no_unguarded_hazards(tmp_path):
             bad += [f"{name}: {w} of {n} wait states\n  {src}\n  {line}" for n, w, src, line in _hazards(body)]
     assert mfma
     assert not bad, f"{len(bad)} unguarded\n" + "\n".join(bad[:20])
+
+
+def test_asm_declares_m0():
+    """An asm statement that writes m0 (the LDS address of a load that goes
+    past the registers) says so, or a value the compiler keeps there is lost."""
+    csrc, n = os.path.join(os.path.dirname(cq.LIB_PATH), "csrc"), 0
+    for f in sorted(os.listdir(csrc)):
+        with open(os.path.join(csrc, f)) as src:
+            for stmt in re.findall(r"\basm\b[^;{]*;", src.read()):
+                if re.search(r"\bs_\w+ m0\b", stmt):
+                    n += 1
+                    assert re.search(r':[^:]*"m0"[^:]*\)\s*;$', stmt), (f, stmt)
+    assert n
