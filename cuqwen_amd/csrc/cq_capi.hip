@@ -112,7 +112,7 @@ extern "C" int cq_compute_logits(int32_t lm_quant, const void* x, const void* W,
   return launch_gemv(a, as_stream(stream));
 }
 
-// Workspace: [epoch uint32, padded to 256 B][stamp uint32 x vocab]; zero it
+// Workspace: [epoch, two uint32, padded to 256 B][stamp uint32 x vocab]; zero it
 // once before the first call.
 extern "C" size_t cq_penalty_workspace_bytes(int32_t vocab) { return 256 + (size_t)(vocab > 0 ? vocab : 0) * 4; }
 

@@ -202,12 +202,14 @@ int launch_rope(__half* q, __half* k, int n_heads, int n_kv, int head_dim, const
                 hipStream_t stream);
 int launch_kv_store(const __half* k, const __half* v, __half* kc, __half* vc, const int* d_pos, int n_kv,
                     int max_seq, int hd, hipStream_t stream);
-// Increments *d_epoch and marks ids d_history[0..*d_history_len) in `stamp` with it.
+// Penalty epoch, two words: marks ids d_history[0..*d_history_len) in `stamp`
+// with d_epoch[0] + 1 and leaves that in d_epoch[1].
 int launch_stamp_history(uint32_t* stamp, const int* d_history, const int* d_history_len, int vocab, uint32_t* d_epoch,
                          hipStream_t stream);
-// Penalty on logits for stamped ids (stand-alone form of the lm_head epilogue).
-int launch_penalty_apply(__half* logits, const uint32_t* stamp, const uint32_t* d_epoch, int vocab,
-                         float penalty, hipStream_t stream);
+// Penalty on logits for ids stamped with d_epoch[1] (stand-alone form of the
+// lm_head epilogue); copies that word to d_epoch[0].
+int launch_penalty_apply(__half* logits, const uint32_t* stamp, uint32_t* d_epoch, int vocab, float penalty,
+                         hipStream_t stream);
 
 // Decode-step control block in device memory.
 struct StepCtl {

@@ -64,43 +64,42 @@ int launch_kv_store(const __half* k, const __half* v, __half* kc, __half* vc, co
 // The reference applies l<0 ? l*p : l/p once per history entry, so repeated
 // ids race and ids past 4096 entries are skipped (kernels.cu:873-905).  Here
 // every distinct id is stamped with the step's epoch and penalised once.
-// One block: the epoch moves on and the history's ids are stamped with it in
-// one launch (with a bump launch of its own in front, logits + penalty +
-// argmax of the 0.5B head took 53.1 instead of 51.6 us).  Bound by its few
-// round trips: eight ids per thread are requested at once, so 32K ids are
-// four batches.
-constexpr int kStampThreads = 1024, kStampBatch = 8;
+// The epoch is two words, so that it moves on without a launch of its own and
+// with blocks in any order: the stamp reads word 0 (the last call's epoch),
+// stamps with the next and leaves it in word 1, which the penalty reads and
+// copies to word 0; neither reads the word that it writes.  Launch bound at any
+// history: 6.9 us a call from 1 to 32768 ids; with a bump launch in front 9.7,
+// and with one block for the whole history, whose barrier does the same, 6.8 up
+// to 4000 ids but 13 at 16000 and 23 at 32768, all its scattered stores leaving
+// one CU.
+constexpr int kStampBlocks = 64, kStampThreads = 256;
 __global__ __launch_bounds__(kStampThreads) void stamp_kernel(uint32_t* stamp, const int* hist, const int* d_len,
                                                               int vocab, uint32_t* d_epoch) {
   const int n = *d_len;
-  const uint32_t ep = *d_epoch + 1u;
-  __syncthreads();   // every thread has read the old epoch
-  if (threadIdx.x == 0) *d_epoch = ep;
-  for (int i0 = threadIdx.x; i0 < n; i0 += kStampThreads * kStampBatch) {
-    int id[kStampBatch];
-#pragma unroll
-    for (int e = 0; e < kStampBatch; ++e) id[e] = hist[min(i0 + e * kStampThreads, n - 1)];
-#pragma unroll
-    for (int e = 0; e < kStampBatch; ++e)
-      if (id[e] >= 0 && id[e] < vocab) stamp[id[e]] = ep;
+  const uint32_t ep = d_epoch[0] + 1u;
+  if (blockIdx.x == 0 && threadIdx.x == 0) d_epoch[1] = ep;
+  for (int i = blockIdx.x * kStampThreads + threadIdx.x; i < n; i += kStampBlocks * kStampThreads) {
+    const int id = hist[i];
+    if (id >= 0 && id < vocab) stamp[id] = ep;
   }
 }
 int launch_stamp_history(uint32_t* stamp, const int* d_history, const int* d_history_len, int vocab, uint32_t* d_epoch,
                          hipStream_t stream) {
-  hipLaunchKernelGGL(stamp_kernel, dim3(1), dim3(kStampThreads), 0, stream, stamp, d_history, d_history_len, vocab,
-                     d_epoch);
+  hipLaunchKernelGGL(stamp_kernel, dim3(kStampBlocks), dim3(kStampThreads), 0, stream, stamp, d_history, d_history_len,
+                     vocab, d_epoch);
   CQ_HIP(hipGetLastError());
   return CQ_OK;
 }
-__global__ void penalty_kernel(_Float16* logits, const uint32_t* stamp, const uint32_t* d_epoch, int vocab,
-                               float penalty) {
+__global__ void penalty_kernel(_Float16* logits, const uint32_t* stamp, uint32_t* d_epoch, int vocab, float penalty) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= vocab || stamp[i] != *d_epoch) return;
+  const uint32_t ep = d_epoch[1];
+  if (i == 0) d_epoch[0] = ep;
+  if (i >= vocab || stamp[i] != ep) return;
   const float pen = (float)(_Float16)penalty;
   const float l = (float)logits[i];
   logits[i] = (_Float16)(l < 0.f ? l * pen : l / pen);
 }
-int launch_penalty_apply(__half* logits, const uint32_t* stamp, const uint32_t* d_epoch, int vocab, float penalty,
+int launch_penalty_apply(__half* logits, const uint32_t* stamp, uint32_t* d_epoch, int vocab, float penalty,
                          hipStream_t stream) {
   hipLaunchKernelGGL(penalty_kernel, dim3((vocab + 255) / 256), dim3(256), 0, stream, (_Float16*)logits, stamp,
                      d_epoch, vocab, penalty);

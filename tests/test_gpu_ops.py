@@ -332,3 +332,20 @@ def test_argmax_and_penalty(g):
     cq.check(cq.lib.cq_apply_repetition_penalty(ld.ptr, g.put(hist), g.i32(hist.size), V, 1.1, pws.ptr, None))
     got = ld.to_array(np.float16)
     assert np.array_equal(got.view(np.uint16), orc.penalty(l, hist).view(np.uint16))
+
+
+def test_penalty_histories_one_after_another(g):
+    """Each call penalises its own history alone, whatever earlier calls on the
+    workspace stamped: empty, one id, around the 64 x 256 threads of the stamp
+    launch, and longer than the vocabulary."""
+    V = 20000
+    rng = np.random.default_rng(5)
+    pws = g.empty(cq.lib.cq_penalty_workspace_bytes(V), zero=True)
+    for n in (700, 0, 1, 16383, 16384, 16385, 40000, 3):
+        hist = rng.integers(-2, V + 2, n).astype(np.int32)
+        l = rng.standard_normal(V).astype(np.float16)
+        ld = g.empty(V * 2)
+        ld.upload(l)
+        cq.check(cq.lib.cq_apply_repetition_penalty(ld.ptr, g.put(hist if n else np.zeros(1, np.int32)), g.i32(n), V, 1.1,
+                                                    pws.ptr, None))
+        assert np.array_equal(ld.to_array(np.float16).view(np.uint16), orc.penalty(l, hist).view(np.uint16)), n
