@@ -100,6 +100,7 @@ def _load():
         "cq_state_last_decode_us": (I32, [P, ctypes.POINTER(ctypes.c_double)]),
         "cq_state_set_attention_mode": (I32, [P, I32]),
         "cq_prefill": (I32, [P, IP, I32, I32, IP]),
+        "cq_state_set_prefill_form": (I32, [P, I32, I32, I32, I32]),
         "cq_state_last_prefill_us": (I32, [P, ctypes.POINTER(ctypes.c_double)]),
         "cq_synth_normal": (ctypes.c_uint16, [U64, U64, U64, F]),
         "cq_synth_uniform": (ctypes.c_uint32, [U64, U64, U64, ctypes.c_uint32]),
@@ -168,7 +169,7 @@ EXPORTED = [
     "cq_last_error", "cq_config_preset", "cq_read_header", "cq_write_synthetic_file", "cq_load_weights",
     "cq_synth_weights", "cq_free_weights", "cq_weights_tensor", "cq_weights_wo_rows", "cq_state_create", "cq_state_destroy",
     "cq_forward", "cq_forward_ex", "cq_decode", "cq_state_logits", "cq_state_fill_kv", "cq_state_kv_read", "cq_state_kv_write",
-    "cq_prefill", "cq_state_last_prefill_us", "cq_state_create_kv", "cq_gqa_attention_decode_kv8",
+    "cq_prefill", "cq_state_set_prefill_form", "cq_state_last_prefill_us", "cq_state_create_kv", "cq_gqa_attention_decode_kv8",
     "cq_gqa_attention_decode_fp8",
     "cq_state_last_decode_us", "cq_state_set_attention_mode", "cq_synth_normal", "cq_synth_uniform", "cq_tensor_stream_id", "cq_kv_stream_id",
     "cq_quantize", "cq_device_count", "cq_malloc", "cq_free", "cq_memcpy_h2d", "cq_memcpy_d2h", "cq_memset", "cq_memcpy_d2d",
@@ -389,6 +390,10 @@ class State:
     def set_attention_mode(self, mode):
         """ATTN_SPLIT (default) or ATTN_WHOLE_CONTEXT (cq_state_set_attention_mode)."""
         check(lib.cq_state_set_attention_mode(self.handle, mode))
+
+    def set_prefill_form(self, gemm_tokens=0, gemm_split=1, attn_rows=0, attn_splits=1):
+        """The form of this state's prefill launches (cq_state_set_prefill_form); 0: by their own rules."""
+        check(lib.cq_state_set_prefill_form(self.handle, gemm_tokens, gemm_split, attn_rows, attn_splits))
 
     def logits(self):
         out = np.zeros(self.cfg.vocab_size, dtype=np.uint16)

@@ -200,6 +200,7 @@ struct cq_state {
   hipEvent_t ev0 = nullptr, ev1 = nullptr;
   double last_us = 0.0;
   double last_prefill_us = 0.0;
+  int pf_want[4] = {0, 1, 0, 1};        // cq_state_set_prefill_form
   // batched-prefill workspace, allocated on the first cq_prefill
   char* pf_arena = nullptr;
   __half *pf_x = nullptr, *pf_a = nullptr, *pf_q = nullptr, *pf_ao = nullptr, *pf_inter = nullptr;
@@ -1028,6 +1029,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       g.rope = s->pf_rope; g.kcache = kc; g.vcache = vc;
       g.kcache8 = kc8; g.vcache8 = vc8; g.kscale = ksc; g.vscale = vsc; g.kv_fmt = s->kv_dtype;
       g.part = s->pf_part; g.part_bytes = kPrefillPartBytes; g.keep_tile = keep_tile;
+      g.want_tokens = s->pf_want[0]; g.want_split = s->pf_want[1];
       CQ_TRY(launch_pf_gemm(g, st));
       PfAttnArgs at;
       at.q = (const _Float16*)s->pf_q; at.kcache = kc; at.vcache = vc; at.out = (_Float16*)s->pf_ao;
@@ -1036,6 +1038,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       at.kcache8 = kc8; at.vcache8 = vc8; at.kscale = ksc; at.vscale = vsc; at.kv_fmt = s->kv_dtype;
       at.int4_layout = c.quant_type == CQ_QUANT_INT4;
       at.part = s->pf_part; at.part_bytes = kPrefillPartBytes;
+      at.want_rows = s->pf_want[2]; at.want_splits = s->pf_want[3];
       CQ_TRY(launch_pf_attention(at, st));
       if (l == c.n_layers - 1) {   // only the last token's row goes on
         if (c0 + M == n) CQ_TRY(prefill_tail(s, M));
@@ -1045,6 +1048,7 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       o.mode = GM_RESID; o.quant = c.quant_type; o.A = (const _Float16*)s->pf_ao; o.M = M; o.N = d; o.K = qd;
       o.W[0] = L.wo; o.S[0] = (const _Float16*)L.so; o.panels = true; o.rows[0] = d; o.out = (_Float16*)s->pf_x;
       o.part = s->pf_part; o.part_bytes = kPrefillPartBytes; o.keep_tile = keep_tile;
+      o.want_tokens = s->pf_want[0]; o.want_split = s->pf_want[1];
       o.norm_w = (const _Float16*)L.post_norm; o.norm_eps = c.norm_eps;
       o.norm_out = (_Float16*)s->pf_a; o.norm_inv = s->pf_inv;
       CQ_TRY(launch_pf_gemm(o, st));
@@ -1054,11 +1058,13 @@ int prefill_batched(cq_state* s, const int32_t* tokens, int n, int pos0) {
       m1.S[0] = (const _Float16*)L.sg; m1.S[1] = (const _Float16*)L.su; m1.rows[0] = I; m1.rows[1] = I;
       m1.out = (_Float16*)s->pf_inter;
       m1.part = s->pf_part; m1.part_bytes = kPrefillPartBytes; m1.keep_tile = keep_tile;
+      m1.want_tokens = s->pf_want[0]; m1.want_split = s->pf_want[1];
       CQ_TRY(launch_pf_gemm(m1, st));
       PfGemmArgs m2;
       m2.mode = GM_RESID; m2.quant = c.quant_type; m2.A = (const _Float16*)s->pf_inter; m2.M = M; m2.N = d; m2.K = I;
       m2.W[0] = L.wd; m2.S[0] = (const _Float16*)L.sd; m2.rows[0] = d; m2.out = (_Float16*)s->pf_x;
       m2.part = s->pf_part; m2.part_bytes = kPrefillPartBytes; m2.keep_tile = keep_tile;
+      m2.want_tokens = s->pf_want[0]; m2.want_split = s->pf_want[1];
       // the next layer's input norm (every layer after this one is still to run)
       m2.norm_w = (const _Float16*)s->w->layers[l + 1].in_norm; m2.norm_eps = c.norm_eps;
       m2.norm_out = (_Float16*)s->pf_a; m2.norm_inv = s->pf_inv;
@@ -1096,6 +1102,19 @@ extern "C" int cq_prefill(cq_state* s, const int32_t* tokens, int32_t n_tokens, 
   CQ_HIP(hipEventElapsedTime(&ms, s->ev0, s->ev1));
   s->last_prefill_us = (double)ms * 1000.0;
   if (token_out) *token_out = s->host_pinned[8];
+  return CQ_OK;
+}
+
+extern "C" int cq_state_set_prefill_form(cq_state* s, int32_t gemm_tokens, int32_t gemm_split, int32_t attn_rows,
+                                         int32_t attn_splits) {
+  if (!s) return fail(CQ_EINVAL, "prefill form: null state");
+  if (gemm_tokens != 0 && gemm_tokens != 16 && gemm_tokens != 32 && gemm_tokens != 64 && gemm_tokens != 128)
+    return fail(CQ_EINVAL, "prefill form: gemm_tokens is 0, 16, 32, 64 or 128");
+  if (attn_rows != 0 && attn_rows != 64 && attn_rows != 128 && attn_rows != 256)
+    return fail(CQ_EINVAL, "prefill form: attn_rows is 0, 64, 128 or 256");
+  if (gemm_split < 1 || gemm_split > 32 || attn_splits < 1 || attn_splits > 64)
+    return fail(CQ_EINVAL, "prefill form: gemm_split outside [1, 32] or attn_splits outside [1, 64]");
+  s->pf_want[0] = gemm_tokens; s->pf_want[1] = gemm_split; s->pf_want[2] = attn_rows; s->pf_want[3] = attn_splits;
   return CQ_OK;
 }
 

@@ -158,6 +158,8 @@ struct PfGemmArgs {
   float* vscale = nullptr;
   int kv_fmt = CQ_KV_INT8;   // CQ_KV_INT8 / CQ_KV_FP8 codes
   bool keep_tile = false;    // always the 128-token tile, split by its rule alone (E4M3 cache: the codes stay the same)
+  int want_tokens = 0;       // 0: the form that pf_plan picks; 16 / 32 / 64: the weight stream, 128: the tile
+  int want_split = 1;        // K ranges of a wanted form
   bool panels = false;       // W[0] / S[0] in 128-column panels (wo_to_panels), not row-major
   // RESID only, optional: RMSNorm of the updated rows (half(x * w) and the scale) into
   // norm_out / norm_inv with weight norm_w
@@ -181,6 +183,8 @@ struct PfAttnArgs {
   // fp32 workspace for the partials of a key range split over blocks (nullptr: no split)
   float* part = nullptr;
   size_t part_bytes = 0;
+  int want_rows = 0;          // 0: pa_plan's pick; else rows per block (64 / 128 / 256)
+  int want_splits = 1;        // key ranges of a wanted form
   int n_rb = 0, splits = 1;   // set by the launcher: row blocks per kv head, key ranges
 };
 // Embedding rows, the RoPE table of positions pos0 .. pos0 + M (`rope`: M *

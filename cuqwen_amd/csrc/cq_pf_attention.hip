@@ -571,6 +571,7 @@ PaPlan pa_plan(const PfAttnArgs& a) {
   const int R = a.M * (a.n_heads / a.n_kv);
   const double tiles_hi = (a.pos0 + a.M + kTileKeys - 1) / kTileKeys, tiles_lo = (double)(a.pos0 + 1) / kTileKeys;
   const size_t row_bytes = (size_t)a.n_kv * R * (a.head_dim + 2) * sizeof(float);   // partials of one range
+  if (a.want_rows) return PaPlan{kPaWaves * 16 * kPaCols / a.want_rows, std::min(a.want_splits, (int)tiles_hi)};
   PaPlan best{1, 1};
   double best_t = 1e30;
   for (int kh = 1; kh <= 4; kh *= 2) {
@@ -627,6 +628,12 @@ int launch_pf_attention(const PfAttnArgs& a, hipStream_t stream) {
   if (a.head_dim != 64 && a.head_dim != 128) return fail(CQ_EINVAL, "prefill attention: head_dim must be 64 or 128");
   if (a.M <= 0 || a.pos0 < 0 || a.pos0 + a.M > a.max_seq) return fail(CQ_ERANGE, "prefill attention: positions");
   if (a.kcache8 && (!a.vcache8 || !a.kscale || !a.vscale)) return fail(CQ_EINVAL, "prefill attention: quantized cache pointers");
+  if (a.want_rows) {
+    if (a.want_rows != 64 && a.want_rows != 128 && a.want_rows != 256)
+      return fail(CQ_EINVAL, "prefill attention: no form with that many rows");
+    if (a.want_splits < 1 || !a.part || (size_t)a.want_splits * a.M * a.n_heads * (a.head_dim + 2) * sizeof(float) > a.part_bytes)
+      return fail(CQ_ERANGE, "prefill attention: the ranges' partials do not fit");
+  }
   return a.head_dim == 128 ? pa_format<128>(a, stream) : pa_format<64>(a, stream);
 }
 

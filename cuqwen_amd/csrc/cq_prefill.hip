@@ -1203,6 +1203,8 @@ static double pf_stream_us(const PfGemmArgs& a, int tt, int S) {
 template <int Q, int MODE>
 static PfPlan pf_plan(const PfGemmArgs& a) {
   const int nks = a.K / kPfK, nmat = MODE == GM_SWIGLU ? 2 : 1;
+  if (a.want_tokens == kPfTok) return PfPlan{0, std::min({a.want_split, kPfMaxSplit, nks})};
+  if (a.want_tokens) return PfPlan{a.want_tokens / 16, MODE == GM_SWIGLU && a.want_split == 1 ? 0 : std::min(a.want_split, nks)};
   PfPlan best{0, pf_tile_split<Q, MODE>(a)};
   // above 1024 tokens the tile is the faster form at every preset's shapes;
   // the stream fetches four scales of a row at a time
@@ -1257,6 +1259,14 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream) {
       return fail(CQ_EINVAL, "prefill gemm: qkv cache pointers");
     if (PfShape<CQ_QUANT_FP16, GM_QKV>::BN % a.head_dim || a.rows[0] % a.head_dim || a.rows[1] % a.head_dim || a.rows[0] + a.rows[1] + a.rows[2] != a.N)
       return fail(CQ_EINVAL, "prefill gemm: qkv rows must be whole heads");
+  }
+  if (a.want_tokens) {
+    if (a.want_tokens != 16 && a.want_tokens != 32 && a.want_tokens != 64 && a.want_tokens != kPfTok)
+      return fail(CQ_EINVAL, "prefill gemm: no form with that many tokens");
+    if (a.want_tokens != kPfTok && a.K / kPfK < 4) return fail(CQ_EINVAL, "prefill gemm: the weight stream needs K of 512");
+    if (a.want_split < 1 || !a.part ||
+        (size_t)a.want_split * (a.mode == GM_SWIGLU ? 2 : 1) * a.M * a.N * sizeof(float) > a.part_bytes)
+      return fail(CQ_ERANGE, "prefill gemm: the split's partials do not fit");
   }
   switch (a.quant) {
     case CQ_QUANT_FP16: return launch_pf_gemm_q<CQ_QUANT_FP16>(a, stream);

@@ -200,9 +200,10 @@ def test_decode_kv8_7b_int4_32k_matches_oracle(fmt):
 @pytest.mark.parametrize("fmt", FMTS)
 @pytest.mark.parametrize("quant,n", [(2, 70), (1, 600), (0, 17)])
 def test_prefill_kv8_matches_oracle(quant, n, fmt):
-    """Batched prefill into a quantized cache (GEMM epilogue quantization,
-    both the split-K and the single-pass epilogue) against the oracle's
-    matching mode run token by token."""
+    """Batched prefill into a quantized cache (rows quantized by the epilogue
+    that the launch picks; tests/test_gpu_prefill_forms.py takes the split and
+    the fused one at the same shape) against the oracle's matching mode run
+    token by token."""
     cfg = tiny_config(quant, max_seq_len=1024)
     w = cq.synth_weights(cfg, 6)
     om = orc.Model.synth(cfg, 6, cfg.max_seq_len)

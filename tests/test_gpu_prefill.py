@@ -76,9 +76,9 @@ def test_prefill_tiny_matches_oracle(quant, segments):
 @pytest.mark.parametrize("heads,kv_heads,hd", [(16, 1, 64), (12, 1, 128), (10, 1, 64), (24, 2, 64)])
 @pytest.mark.parametrize("quant", [0, 2])
 def test_prefill_large_gqa_groups_match_oracle(quant, heads, kv_heads, hd):
-    """GQA groups of 9-16 query heads per kv head (the per-head prefill
-    attention path for the fp16 cache) against the oracle run token by
-    token: logits, top-1 and the KV cache, then decode continues."""
+    """GQA groups of 9-16 query heads per kv head (more rows of a token than
+    a 16-row slice has, or not a multiple of it) against the oracle run token
+    by token: logits, top-1 and the KV cache, then decode continues."""
     cfg = tiny_config(quant, n_heads=heads, n_kv_heads=kv_heads, head_dim=hd, dim=1024)
     w = cq.synth_weights(cfg, 23)
     om = orc.Model.synth(cfg, 23, cfg.max_seq_len)
@@ -133,8 +133,8 @@ def _gpu_reference(cfg, w, prompt, pos0, n_ctx):
 def test_prefill_matches_decode_real_shapes(model, quant, layers, n, n_ctx):
     """BASELINE model shapes: batched prefill equals the decode step run once
     per prompt token (logits within 1e-2, same top-1 where the top-2 gap
-    exceeds 1e-2, same KV cache within 1e-2).  Short prompts take the split-K
-    GEMM path, the 2100-token one the single-pass epilogues."""
+    exceeds 1e-2, same KV cache within 1e-2), in the forms that the launches
+    pick for these shapes (tests/test_gpu_prefill_forms.py: every form)."""
     cfg = cq.preset(model, quant).replace(n_layers=layers)
     w = cq.synth_weights(cfg, 0x5157454E)
     prompt = _prompt(cfg, n, 31)
@@ -154,9 +154,10 @@ def test_prefill_matches_decode_real_shapes(model, quant, layers, n, n_ctx):
 
 
 # query rows (n * group) around the 32-row waves and the 64 / 128 / 256-row
-# blocks, contexts around the 32-key tiles and long enough for split key
-# ranges (2 tokens at 3001: more ranges than a block has waves), every cache
-# format, both head sizes, groups that do not divide a wave
+# blocks (256 only at contexts of a few tiles: tests/test_gpu_prefill_forms.py
+# has each block size over long ones), contexts around the 32-key tiles and long
+# enough for split key ranges (2 tokens at 3001: more ranges than a block has
+# waves), every cache format, both head sizes, groups that do not divide a wave
 @pytest.mark.parametrize("heads,kv_heads,hd,n,pos0", [
     (14, 2, 64, 9, 0), (14, 2, 64, 37, 31), (14, 2, 64, 5, 1000), (16, 16, 64, 33, 0), (28, 4, 128, 2, 3001),
     (28, 4, 128, 10, 0), (28, 4, 128, 37, 95), (12, 1, 128, 11, 700), (16, 1, 128, 17, 33), (5, 5, 128, 64, 32)])
