@@ -571,7 +571,10 @@ PaPlan pa_plan(const PfAttnArgs& a) {
   const int R = a.M * (a.n_heads / a.n_kv);
   const double tiles_hi = (a.pos0 + a.M + kTileKeys - 1) / kTileKeys, tiles_lo = (double)(a.pos0 + 1) / kTileKeys;
   const size_t row_bytes = (size_t)a.n_kv * R * (a.head_dim + 2) * sizeof(float);   // partials of one range
-  if (a.want_rows) return PaPlan{kPaWaves * 16 * kPaCols / a.want_rows, std::min(a.want_splits, (int)tiles_hi)};
+  if (a.want_rows) {
+    const int most = (int)std::min<size_t>((size_t)tiles_hi, a.part_bytes / row_bytes);
+    return PaPlan{kPaWaves * 16 * kPaCols / a.want_rows, std::max(std::min(a.want_splits, most), 1)};
+  }
   PaPlan best{1, 1};
   double best_t = 1e30;
   for (int kh = 1; kh <= 4; kh *= 2) {
@@ -631,8 +634,7 @@ int launch_pf_attention(const PfAttnArgs& a, hipStream_t stream) {
   if (a.want_rows) {
     if (a.want_rows != 64 && a.want_rows != 128 && a.want_rows != 256)
       return fail(CQ_EINVAL, "prefill attention: no form with that many rows");
-    if (a.want_splits < 1 || !a.part || (size_t)a.want_splits * a.M * a.n_heads * (a.head_dim + 2) * sizeof(float) > a.part_bytes)
-      return fail(CQ_ERANGE, "prefill attention: the ranges' partials do not fit");
+    if (a.want_splits < 1 || (a.want_splits > 1 && !a.part)) return fail(CQ_EINVAL, "prefill attention: key ranges");
   }
   return a.head_dim == 128 ? pa_format<128>(a, stream) : pa_format<64>(a, stream);
 }

@@ -1140,7 +1140,7 @@ static int launch_pf_tile(const PfGemmArgs& a, int S, hipStream_t stream) {
 // 0: PS_SWIGLU), or, tt = 0, the 128-token tile (split ways, 1: unsplit).
 struct PfPlan { int tt, split; };
 
-// The tile's split for more than 256 tokens.  Model: one block fits a CU (its
+// The tile's split for more than 512 tokens.  Model: one block fits a CU (its
 // LDS), so B blocks take ceil(B / CUs) rounds and S splits ceil(S B / CUs)
 // rounds of 1/S the work; a full-K block runs at ~4.2 TFLOP/s per CU
 // (measured: int4 gate/up, 56 us per round of 256 blocks at K = 3584); the
@@ -1170,55 +1170,74 @@ static int pf_tile_split(const PfGemmArgs& a) {
   return S;
 }
 
-// Microseconds of either form, fitted to 5,000 measured (model, precision,
-// GEMM, tokens 8 .. 777, form, split) points; rms error 15 %, and the picks
-// cost 2 % (stream) and 4 % (tile) over the best of each form on average.
-// Tile: rounds of one block per CU, each a fixed part and its K steps.
-// Stream: the K steps of a wave times the blocks on the fullest CU.  Both: a
-// launch and the partials' bytes (written and read) for a split epilogue.
+// Microseconds of either form, fitted to 54,000 measured points: the five
+// presets' four GEMMs, three precisions, 36 token counts from 2 to 1024, every
+// token tile and split, 2 us added for a launch of the epilogue's own; rms error
+// 6 %.  What is picked by it costs 0.7 % over the best measured form on average;
+// nine of 2104 shapes are over 2 % behind the tile by the split rule above alone
+// (one by 7.5 %, the rest under 4.2), no layer's four GEMMs together over 0.8.
+// Tile: rounds of one block per CU, each with its K steps, and the split
+// epilogue with the partials written and read, or the fused one.
+// Stream: the K steps of a wave on the fullest CU, the blocks after the first
+// there, and the fused SwiGLU of each or the split epilogue.
+// Both: the weights' bytes once.  (Without that term, and with no cost of its
+// own for the fused SwiGLU, the stream was up to 25 % too cheap and was picked
+// for gate/up where the tile is faster: 14B int8 at 288 tokens 192 against 161
+// us, 7B int8 at 256 141 against 122.)
+template <int Q> constexpr double pf_by(double int4, double int8, double fp16) {
+  return Q == CQ_QUANT_INT4 ? int4 : Q == CQ_QUANT_INT8 ? int8 : fp16;
+}
 template <int Q, int MODE>
 static double pf_tile_us(const PfGemmArgs& a, int S) {
-  constexpr double kFixed = Q == CQ_QUANT_FP16 ? 11.5 : 9.5, kStep = Q == CQ_QUANT_INT4 ? 1.6 : Q == CQ_QUANT_INT8 ? 1.85 : 2.6;
+  constexpr double kRound = pf_by<Q>(0.1, 0.46, 0.48), kStep = pf_by<Q>(1.6, 1.84, 2.57);
+  constexpr double kSplit = pf_by<Q>(11.4, 11.4, 12.3), kPerMb = pf_by<Q>(0.39, 0.39, 0.365);
   const int bn = PfShape<Q, MODE>::BN, nmat = MODE == GM_SWIGLU ? 2 : 1, nks = a.K / kPfK;
   const int64_t blocks = (int64_t)((a.N + bn - 1) / bn) * ((a.M + kPfTok - 1) / kPfTok) * S;
-  const double mb = (double)S * nmat * a.M * a.N * sizeof(float) / 1e6;
-  const double per_mb = a.M > 256 ? 0.42 : 0.6;   // larger partials stream better
-  return -2.0 + (double)((blocks + kNumCUs - 1) / kNumCUs) * (kFixed + (nks + S - 1) / S * kStep) +
-         (S > 1 ? 2.3 + per_mb * mb : MODE == GM_QKV ? 18.0 : 0.0);
+  const double rounds = (double)((blocks + kNumCUs - 1) / kNumCUs), mb = (double)S * nmat * a.M * a.N * sizeof(float) / 1e6;
+  const double weight_mb = (double)nmat * a.N * a.K * pf_by<Q>(0.5, 1, 2) / 1e6;
+  const double fused = MODE == GM_QKV      ? pf_by<Q>(19.6, 19.7, 19.9)
+                       : MODE == GM_SWIGLU ? pf_by<Q>(6.9, 5.7, 4.8) * rounds
+                                           : pf_by<Q>(13.3, 12.7, 14.2);
+  return pf_by<Q>(0.051, 0.055, 0.057) * weight_mb + rounds * (kRound + (nks + S - 1) / S * kStep) +
+         (S > 1 ? kSplit + kPerMb * mb : fused);
 }
 template <int Q>
 static double pf_stream_us(const PfGemmArgs& a, int tt, int S) {
-  constexpr double kFixed = Q == CQ_QUANT_INT4 ? 5.0 : Q == CQ_QUANT_INT8 ? 6.3 : 7.8;
-  constexpr double kStep[3] = {Q == CQ_QUANT_INT4 ? 0.70 : Q == CQ_QUANT_INT8 ? 1.13 : 2.1,
-                               Q == CQ_QUANT_INT4 ? 0.87 : Q == CQ_QUANT_INT8 ? 1.2 : 2.27,
-                               Q == CQ_QUANT_INT4 ? 1.14 : Q == CQ_QUANT_INT8 ? 1.44 : 2.45};
-  constexpr double kRound = Q == CQ_QUANT_FP16 ? 3.8 : 2.1;
+  constexpr double kStep[3] = {pf_by<Q>(0.584, 1.12, 1.87), pf_by<Q>(0.784, 1.13, 2.14), pf_by<Q>(1.066, 1.37, 2.39)};
+  constexpr double kBlock[3] = {pf_by<Q>(2.25, 2.2, 3.8), pf_by<Q>(2.38, 2.6, 3.7), pf_by<Q>(3.3, 3.3, 4.2)};
+  constexpr double kSwiglu[3] = {pf_by<Q>(0.26, 0.11, 0.2), pf_by<Q>(0.95, 0.96, 0.85), pf_by<Q>(1.26, 1.95, 1.18)};
   const int rows = a.rows[0] + a.rows[1] + a.rows[2], s = std::max(S, 1), nks = a.K / kPfK;
   const int64_t blocks = (int64_t)((rows + kPsRows - 1) / kPsRows) * ((a.M + 16 * tt - 1) / (16 * tt)) * s;
   const double per_cu = (double)((blocks + kNumCUs - 1) / kNumCUs), steps = ((nks + s - 1) / s + 1) / 2;
-  return kFixed + steps * kStep[tt / 2] * per_cu + kRound * (per_cu - 1) +
-         (S ? 3.5 + 0.57 * S * a.M * (double)rows * sizeof(float) / 1e6 : 0.0);
+  const double weight_mb = (double)rows * a.K * pf_by<Q>(0.5, 1, 2) / 1e6, mb = (double)S * a.M * rows * sizeof(float) / 1e6;
+  return pf_by<Q>(3.73, 3.88, 4.47) + pf_by<Q>(0.077, 0.066, 0.061) * weight_mb + steps * kStep[tt / 2] * per_cu +
+         kBlock[tt / 2] * (per_cu - 1) +
+         (S ? pf_by<Q>(7.0, 7.5, 8.4) + pf_by<Q>(0.334, 0.38, 0.357) * mb : kSwiglu[tt / 2] * per_cu);
 }
 
 template <int Q, int MODE>
 static PfPlan pf_plan(const PfGemmArgs& a) {
   const int nks = a.K / kPfK, nmat = MODE == GM_SWIGLU ? 2 : 1;
-  if (a.want_tokens == kPfTok) return PfPlan{0, std::min({a.want_split, kPfMaxSplit, nks})};
-  if (a.want_tokens) return PfPlan{a.want_tokens / 16, MODE == GM_SWIGLU && a.want_split == 1 ? 0 : std::min(a.want_split, nks)};
+  if (a.want_tokens) {
+    const int most = (int)std::min<size_t>(nks, a.part_bytes / ((size_t)nmat * a.M * a.N * sizeof(float)));
+    if (a.want_tokens == kPfTok) return PfPlan{0, std::min({a.want_split, kPfMaxSplit, most})};
+    const int s = std::min(a.want_split, most);
+    return PfPlan{a.want_tokens / 16, MODE == GM_SWIGLU && s == 1 ? 0 : s};
+  }
   PfPlan best{0, pf_tile_split<Q, MODE>(a)};
   // above 1024 tokens the tile is the faster form at every preset's shapes;
   // the stream fetches four scales of a row at a time
   if (a.keep_tile || !a.part || a.M > 1024 || nks < 4) return best;
   auto fits = [&](int s) { return (size_t)s * nmat * a.M * a.N * sizeof(float) <= a.part_bytes; };
-  if (a.M <= 256) {
+  // up to 512 tokens the fitted split is as good as the rule's or better (above,
+  // not always: 3B int4 QKV at 1024 33 against 31 us)
+  if (a.M <= 512) {
     for (int s = 1; s <= std::min(kPfMaxSplit, nks) && (s == 1 || fits(s)); ++s)
       if (s == 1 || pf_tile_us<Q, MODE>(a, s) < pf_tile_us<Q, MODE>(a, best.split)) best.split = s;
   }
-  // the stream has to win by some of the model's error (where it errs for the
-  // stream: 0.5B int4 gate/up at 1000 tokens 42 against 36 us, 7B int4 QKV at
-  // 1024 78 against 68)
-  const double margin = a.M <= 512 ? 0.97 : MODE == GM_SWIGLU ? 0.88 : 0.95;
-  double t = margin * pf_tile_us<Q, MODE>(a, best.split);
+  // above 512 tokens partials make the stream err by more: it has to win by that
+  // (0.5B fp16 down at 704 32 against 29 us without)
+  double t = (a.M <= 512 || MODE == GM_SWIGLU ? 1.0 : 0.95) * pf_tile_us<Q, MODE>(a, best.split);
   for (int tt = 1; tt <= 4; tt *= 2)
     for (int s = MODE == GM_SWIGLU ? 0 : 1; s <= std::min(32, nks) && fits(s); ++s)
       if (const double u = pf_stream_us<Q>(a, tt, s); u < t) {
@@ -1264,9 +1283,8 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream) {
     if (a.want_tokens != 16 && a.want_tokens != 32 && a.want_tokens != 64 && a.want_tokens != kPfTok)
       return fail(CQ_EINVAL, "prefill gemm: no form with that many tokens");
     if (a.want_tokens != kPfTok && a.K / kPfK < 4) return fail(CQ_EINVAL, "prefill gemm: the weight stream needs K of 512");
-    if (a.want_split < 1 || !a.part ||
-        (size_t)a.want_split * (a.mode == GM_SWIGLU ? 2 : 1) * a.M * a.N * sizeof(float) > a.part_bytes)
-      return fail(CQ_ERANGE, "prefill gemm: the split's partials do not fit");
+    if (a.want_split < 1 || !a.part || (size_t)(a.mode == GM_SWIGLU ? 2 : 1) * a.M * a.N * sizeof(float) > a.part_bytes)
+      return fail(CQ_ERANGE, "prefill gemm: the partials do not fit");
   }
   switch (a.quant) {
     case CQ_QUANT_FP16: return launch_pf_gemm_q<CQ_QUANT_FP16>(a, stream);

@@ -430,11 +430,11 @@ int cq_dequantize(int32_t quant_type, int32_t group_size, const void* W, const v
  * stream's tile; K of at least 512) or 128 (the large tile), its K cut into
  * gemm_split ranges (at most the K steps; 8 for the large tile); attn_rows 64,
  * 128 or 256 (query rows per attention block), the keys cut into attn_splits
- * ranges (at most the 32-key tiles; an E4M3 cache has one form).  0 in
- * gemm_tokens or attn_rows: by the rules again.  A prefill whose partials do
- * not fit the state's workspace then returns CQ_ERANGE.  Test hook, so that
- * every form is checked at shapes that the rules would give to another; no
- * counterpart in the reference. */
+ * ranges (at most the 32-key tiles; an E4M3 cache has one form).  Ranges are
+ * further limited to those whose partials fit the state's workspace.  0 in
+ * gemm_tokens or attn_rows: by the rules again.  Test hook, so that every form
+ * is checked at shapes that the rules would give to another; no counterpart in
+ * the reference. */
 int cq_state_set_prefill_form(cq_state* s, int32_t gemm_tokens, int32_t gemm_split, int32_t attn_rows,
                               int32_t attn_splits);
 
