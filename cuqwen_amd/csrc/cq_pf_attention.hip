@@ -13,19 +13,20 @@
 // Where rows and key groups leave CUs idle the key range is also cut over S
 // blocks, whose fp32 partials a second launch merges (pa_plan).
 //
-// What bounds it: at long contexts the matrix cores under the part's power
-// limit (7B heads, 2048 tokens after 30720, fp16 cache: 1.03-1.11 ms a layer,
-// 840-910 TFLOP/s; with the exponentials, the LDS reads, the staging and the
-// barriers all taken out the same loop still takes 0.90-0.95, and bare matrix
-// instructions on random operands reach 1.9 PFLOP/s); at short ones the chain
-// of launch, first loads, a few steps and the epilogue (7 us).  Why this
-// shape: one head per wave and 16 rows per wave made each K / V fragment feed
-// one instruction and left LDS and the softmax arithmetic in front (1.86 ms);
-// 32 rows per wave 1.31, the score and value products overlapped with the
-// softmax of the neighbouring step 1.19, requests straight into LDS two steps
-// ahead 1.03.  7B heads: 1024 tokens 36 -> 24 us; 27 tokens after 1500, whose
-// 8 blocks once walked the whole context, 45 -> 16 us.  The scores stay in
-// 32 bits up to the exponent (the decode step rounds them to fp16).
+// What bounds it: at long contexts matrix units that wait (7B heads, 2048
+// tokens after 30720, fp16 cache, KH = 2: 1.03-1.11 ms a layer, 840-910
+// TFLOP/s, the units busy 40 % of the active cycles; with the exponentials, the
+// LDS reads, the staging and the barriers all taken out the same loop took
+// 0.90-0.95) and power (on a cache of zeros 0.87 against 1.08 ms, the clock at
+// 2.08 of 2.4 GHz on random values); at short ones the chain of launch, first
+// loads, a few steps and the epilogue (7 us).  Why this shape: one head per
+// wave and 16 rows per wave made each K / V fragment feed one instruction and
+// left LDS and the softmax arithmetic in front (1.86 ms); 32 rows per wave
+// 1.31, the score and value products overlapped with the softmax of the
+// neighbouring step 1.19, requests straight into LDS 1.03.  7B heads: 1024
+// tokens 36 -> 26 us; 27 tokens after 1500, whose 8 blocks once walked the whole
+// context, 45 -> 16 us.  The scores stay in 32 bits up to the exponent (the
+// decode step rounds them to fp16).
 #include "cq_attention.h"
 #include "cq_prefill.h"
 
@@ -47,7 +48,8 @@ struct PaShape {
   static constexpr int TPS = KH * TPW;                  // tiles per step
   static constexpr int TILE = kTileKeys * HD;           // halves of K (or V) per tile
   static constexpr int STAGE = 2 * TPS * TILE;          // halves: K tiles, then V tiles
-  // LDS slots: three (requests two steps ahead) where they fit
+  // LDS slots: three (requests two steps ahead) where they fit 96 KB, that is
+  // with KH = 1 and, at head size 64, 2; else two (one step ahead)
   static constexpr int NS = KV8 == 0 && 3 * STAGE * 2 <= 96 * 1024 ? 3 : 2;
   static constexpr int DT = HD / 16;
   static constexpr int STATE = kPaCols * (2 + 4 * DT);  // floats of one lane's softmax state (whole f4_t)

@@ -658,9 +658,11 @@ __global__ __launch_bounds__(kPfThreads, 2) void pf_gemm_kernel(const PfGemmArgs
 // loads complete in issue order per wave, so a wave that requested both would
 // wait for weights of later steps whenever it needs activations.
 // What bounds it: each wave's step (unpack, LDS reads, matrix instructions,
-// a barrier) and the weight bytes about equally.  7B int4 gate/up at 27
-// tokens 34.6 us = 2.0 TB/s; with the weight loads alone 20, with everything
-// but them 21-25.  The 128-token tile it replaces there does the work of 128
+// a barrier) and the weight bytes about equally, not overlapped as they should
+// be: D steps of weights are requested ahead, but the step's branches make the
+// compiler wait for all of them at the first of every four steps.  7B int4
+// gate/up at 27 tokens 34.6 us = 2.0 TB/s; with the weight loads alone 20, with
+// everything but them 21-25.  The 128-token tile it replaces there does the work of 128
 // tokens: 69 us as it was split, 54 unsplit; down 43 -> 22, QKV 18 -> 13, O
 // 16 -> 11 (with their epilogues).  0.5B int4 at 27 tokens: gate/up 37 -> 7.
 // Measured on the way: four scales per load instead of one 28 -> 22 us (8
@@ -675,7 +677,7 @@ constexpr int kPsWaves = kPsRG * kPsKG, kPsThreads = (kPsWaves + 1) * kWave;
 constexpr int kPsRows = kPsRG * 32;
 constexpr int kPsUnroll = 4;   // steps per loop iteration: scales are fetched four groups at a time
 template <int Q, int TT> struct PsShape {
-  static constexpr int D = Q == CQ_QUANT_INT4 ? 4 : 2;   // weight steps in flight
+  static constexpr int D = Q == CQ_QUANT_INT4 ? 4 : 2;   // weight steps requested ahead
   static constexpr int NST = TT == 4 ? 3 : 4;            // stages
   static constexpr int XT = 16 * TT * kPfK;              // halves of one step's activations
   static constexpr int XS = kPsKG * XT;                  // a stage: one step of each K group

@@ -187,7 +187,10 @@ int cq_decode(cq_state* s, int32_t token, int32_t pos0, int32_t n_steps,
  * tokens per pass), the last layer's O-proj / MLP and the lm_head run for the
  * last token only (a one-token prompt is a plain decode step).  Fills the
  * KV cache for positions [pos0, pos0 + n_tokens); *token_out receives the
- * greedy id after the last prompt token and cq_state_logits its logits.
+ * greedy id after the last prompt token and cq_state_logits its logits.  The
+ * state's first prompt allocates its working memory, held until the state is
+ * freed: 128 MB of partial sums and 2048 tokens' activations (2 dim, 2 n_heads *
+ * head_dim and intermediate_size halves each; 7B: 259 MB in all).
  * Errors: CQ_ERANGE for positions past max_seq_len or ids outside the
  * vocabulary. */
 int cq_prefill(cq_state* s, const int32_t* tokens, int32_t n_tokens, int32_t pos0, int32_t* token_out);
