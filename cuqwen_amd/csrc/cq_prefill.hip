@@ -1160,8 +1160,9 @@ static int pf_tile_split(const PfGemmArgs& a) {
     const double t1 = (double)bn * nmat * kPfTok * a.K * 2 / 4.2e6;     // us, one round of full-K blocks
     const double part_us = (double)nmat * a.M * a.N * sizeof(float) / 2.8e6;   // us per split of partials
     // QKV's unsplit epilogue (RoPE through an LDS tile, cache stores) costs
-    // about what a split epilogue's pass does (measured: 7B at 1024 tokens 72
-    // us unsplit, 67 split 3 ways; at 1536 71 and 100)
+    // about what a split epilogue's pass does (measured: 7B at 1024 tokens 75
+    // us unsplit, 72 split 3 ways; at 1536 72 and 100, at 2048 136 and 125
+    // split 2 ways)
     double best = rounds(1) * t1 + (MODE == GM_QKV ? part_us + 2.0 : 0.0);
     for (int s = 2; s <= std::min(kPfMaxSplit, nks); ++s) {
       if ((size_t)s * nmat * a.M * a.N * sizeof(float) > (a.keep_tile ? std::min(a.part_bytes, kPfKeptPart) : a.part_bytes)) break;
@@ -1222,9 +1223,9 @@ static PfPlan pf_plan(const PfGemmArgs& a) {
   const int nks = a.K / kPfK, nmat = MODE == GM_SWIGLU ? 2 : 1;
   if (a.want_tokens) {
     const int most = (int)std::min<size_t>(nks, a.part_bytes / ((size_t)nmat * a.M * a.N * sizeof(float)));
-    if (a.want_tokens == kPfTok) return PfPlan{0, std::min({a.want_split, kPfMaxSplit, most})};
+    if (a.want_tokens == kPfTok) return PfPlan{0, std::max(std::min({a.want_split, kPfMaxSplit, most}), 1)};
     const int s = std::min(a.want_split, most);
-    return PfPlan{a.want_tokens / 16, MODE == GM_SWIGLU && s == 1 ? 0 : s};
+    return PfPlan{a.want_tokens / 16, MODE == GM_SWIGLU && s <= 1 ? 0 : s};
   }
   PfPlan best{0, pf_tile_split<Q, MODE>(a)};
   // above 1024 tokens the tile is the faster form at every preset's shapes;
@@ -1285,8 +1286,9 @@ int launch_pf_gemm(const PfGemmArgs& a, hipStream_t stream) {
     if (a.want_tokens != 16 && a.want_tokens != 32 && a.want_tokens != 64 && a.want_tokens != kPfTok)
       return fail(CQ_EINVAL, "prefill gemm: no form with that many tokens");
     if (a.want_tokens != kPfTok && a.K / kPfK < 4) return fail(CQ_EINVAL, "prefill gemm: the weight stream needs K of 512");
-    if (a.want_split < 1 || !a.part || (size_t)(a.mode == GM_SWIGLU ? 2 : 1) * a.M * a.N * sizeof(float) > a.part_bytes)
-      return fail(CQ_ERANGE, "prefill gemm: the partials do not fit");
+    if (a.want_split < 1 || !a.part) return fail(CQ_EINVAL, "prefill gemm: a wanted form needs a split and the workspace");
+    if (a.want_tokens != kPfTok && a.mode != GM_SWIGLU && (size_t)a.M * a.N * sizeof(float) > a.part_bytes)
+      return fail(CQ_ERANGE, "prefill gemm: the weight stream's partials do not fit");
   }
   switch (a.quant) {
     case CQ_QUANT_FP16: return launch_pf_gemm_q<CQ_QUANT_FP16>(a, stream);
